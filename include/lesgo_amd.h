@@ -231,7 +231,7 @@ enum {
     LG_K_ROWS_C2R = 1,          /* inverse rows, nx points */
     LG_K_COLS_FWD = 2,          /* forward columns, ny points */
     LG_K_COLS_INV = 3,          /* inverse columns, ny points */
-    LG_K_TRIDAG = 4,            /* pressure tridiagonal */
+    LG_K_TRIDAG = 4,            /* pressure solve (spectral step: the whole column pass) */
     LG_K_ROWS_R2C_PAD = 5,      /* forward rows on the 3/2 grid */
     LG_K_ROWS_C2R_PAD = 6,      /* inverse rows on the 3/2 grid */
     LG_K_COLS_UNPAD = 7,        /* forward columns, 3/2 grid to nx x ny */

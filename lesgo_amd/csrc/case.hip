@@ -12,6 +12,7 @@
 
 #include "case.hpp"
 #include "clock.hpp"
+#include "column.hpp"
 #include "passes.hpp"
 #include "lagrange.hpp"
 #include "pointwise.hpp"
@@ -178,14 +179,40 @@ Case<T>::Case(const lg_params& p, int members) : d(p), M(members), Ma(members) {
     mbsp = (long)(d.nz + 1) * d.bsplane;
     LG_HIP(hipStreamCreate(&stream));
     for (int i = 0; i < LG_NFIELDS; ++i) fld[i] = dalloc<T>(M * d.field);
-    for (int i = 0; i < NSPEC; ++i) spec[i] = dalloc<cplx<T>>(M * msp);
+    cfl_mode = p.use_cfl_dt != 0;
+    // a CFL step reads the end-of-step velocity at its head, so only fixed-dt
+    // cases keep the spectra between steps; LESGO_AMD_PHYSICAL_STEP=1 in the
+    // environment keeps every case on the all-physical step
+    const char* phys = std::getenv("LESGO_AMD_PHYSICAL_STEP");
+    spec_on = !cfl_mode && !(phys && phys[0] == '1');
+    {
+        // the spectra in one allocation: a thread of the column pass reads all
+        // of them level by level, and fewer address translations miss when
+        // they lie together (256 x 256 x 192 FP32: 286 against 300 us apart)
+        spool = dalloc<cplx<T>>((NSPEC + 3 + (spec_on ? 12 : 0)) * M * msp);
+        cplx<T>* q = spool;
+        auto take = [&] {
+            cplx<T>* r = q;
+            q += M * msp;
+            return r;
+        };
+        for (int i = 0; i < NSPEC; ++i) spec[i] = take();
+        sU = take();
+        sV = take();
+        sW = take();
+        if (spec_on) {
+            for (int i = 0; i < 3; ++i) sR[i] = take();
+            for (int i = 0; i < 3; ++i) sRf[i] = take();
+            for (int i = 0; i < 3; ++i) sF[i] = take();
+            sP = take();
+            sPf = take();
+            sDz = take();
+        }
+    }
     prod_fused = prod_fused_for(d.nx2, d.ny2, (int)sizeof(T));
     for (int i = 0; i < (prod_fused ? 6 : NBIG); ++i) big[i] = dalloc<T>(M * mbp);
     for (int i = 0; i < 6; ++i) bigspec[i] = dalloc<cplx<T>>(M * mbsp);
     for (int i = 0; i < NTMP; ++i) tmp[i] = dalloc<T>(M * d.field);
-    sU = dalloc<cplx<T>>(M * msp);
-    sV = dalloc<cplx<T>>(M * msp);
-    sW = dalloc<cplx<T>>(M * msp);
     gam = dalloc<double>(msp);
     {
         // the elimination coefficients of the pressure systems (grid only)
@@ -217,27 +244,16 @@ Case<T>::Case(const lg_params& p, int members) : d(p), M(members), Ma(members) {
     d_flags = dalloc<int>(6L * M);
     mcold.assign(M, 1);
     rhsf_phys.assign(M, 1);
-    cfl_mode = p.use_cfl_dt != 0;
     d_clock = dalloc<double>((long)CK_N * M);
     d_cmax = dalloc<unsigned long long>(3L * M);
     mtime.assign(M, 0.0);
     clk_fresh.assign(M, 1);
     for (int m = 0; m < M; ++m) clock_reset(m);
-    // a CFL step reads the end-of-step velocity at its head, so only fixed-dt
-    // cases keep the spectra between steps; LESGO_AMD_PHYSICAL_STEP=1 in the
-    // environment keeps every case on the all-physical step
-    const char* phys = std::getenv("LESGO_AMD_PHYSICAL_STEP");
-    spec_on = !cfl_mode && !(phys && phys[0] == '1');
     if (spec_on) {
         for (int q = 0; q < 3; ++q) {
-            sR[q] = dalloc<cplx<T>>(M * msp);
-            sRf[q] = dalloc<cplx<T>>(M * msp);
-            sF[q] = dalloc<cplx<T>>(M * msp);
             fprev[q] = dalloc<T>(M * d.field);
             tprev[q] = dalloc<T>(M * d.field);
         }
-        sP = dalloc<cplx<T>>(M * msp);
-        sDz = dalloc<cplx<T>>(M * msp);
     }
     px.build(d.nx);
     py.build(d.ny);
@@ -288,13 +304,10 @@ Case<T>::~Case() {
         if (p) (void)hipFree(p);
     };
     for (auto p : fld) fr(p);
-    for (auto p : spec) fr(p);
+    fr(spool);
     for (auto p : big) fr(p);
     for (auto p : bigspec) fr(p);
     for (auto p : tmp) fr(p);
-    fr(sU);
-    fr(sV);
-    fr(sW);
     fr(gam);
     fr(usc);
     fr(dev_err);
@@ -309,14 +322,9 @@ Case<T>::~Case() {
     fr(d_clock);
     fr(d_cmax);
     for (int q = 0; q < 3; ++q) {
-        fr(sR[q]);
-        fr(sRf[q]);
-        fr(sF[q]);
         fr(fprev[q]);
         fr(tprev[q]);
     }
-    fr(sP);
-    fr(sDz);
     fr(tavg);
     fr(tspec);
     fr(G1);
@@ -470,7 +478,7 @@ size_t case_bytes(const lg_params& p, int members, int tsize) {
          21 * M * chunk * d.splane * 2 * T;
     b += 3 * M * sizeof(double) + 1024 * sizeof(double) + 2 * d.splane * T;
     b += M * (CK_N * sizeof(double) + 3 * sizeof(unsigned long long) + 2 * sizeof(int));
-    if (!p.use_cfl_dt) b += 11 * M * msp * 2 * T + 6 * M * d.field * T;   // spectral state
+    if (!p.use_cfl_dt) b += 12 * M * msp * 2 * T + 6 * M * d.field * T;   // spectral state
     return b;
 }
 
@@ -650,6 +658,12 @@ void Case<T>::cols_unpad(int njobs, cplx<T>* const* dst, int lev0, int nlev) {
 // ---------------------------------------------------------------------------
 // Small helpers
 // ---------------------------------------------------------------------------
+template <typename T>
+static SpecGeo<T> spec_geo(const Dims& d, long msp, int k0, int nlev) {
+    return SpecGeo<T>{d.ny, d.NK, d.nz, k0, nlev, d.splane, msp, (T)(2.0 * PI_D / d.prm.lx),
+                      (T)(2.0 * PI_D / d.prm.ly)};
+}
+
 #define GEO(k0, nlev) (Geo{d.nx, d.ny, d.nz, d.ld, d.plane, (k0), (nlev), d.field})
 
 static inline dim3 grid_ij(int W, int ny, int nlev, int M) {
@@ -1290,12 +1304,14 @@ void Case<T>::press_stag_array() {
     }
     TriGeo tg{d.ny, d.NK, d.nz, d.splane, msp, Ma, 2.0 * PI_D / d.prm.lx,
               2.0 * PI_D / d.prm.ly, d.dz, 1.0 / (d.dz * d.dz), 1.0 / d.dz};
-    const int nsys = Ma * d.ny * d.NK;
     const double tbytes =
         (double)Ma * d.splane * sizeof(cplx<T>) * (3.0 * d.nz + 1 + 2 + d.nz + 1);
-    const PassChoice ch = choice_for<T>(PK_TRIDAG, d.ny, d.NK);
-    const int tb = ch.S;
     timer.run(stream, KK_TRIDAG, tbytes, [&] {
+        const ColPress<T> cp{spec[0], spec[1], spec[2], spec[3], spec[3] + d.splane};
+        if (launch_column<T, false>(SpecAb2<T>{}, cp, spec_geo<T>(d, msp, 1, d.nz), tg, spec[4],
+                                    gam, (T)d.dz, dev_err, Ma, stream))
+            return;
+        const int nsys = Ma * d.ny * d.NK, tb = choice_for<T>(PK_TRIDAG, d.ny, d.NK).S;
         LG_LAUNCH(k_tridag<T>, dim3((nsys + tb - 1) / tb), dim3(tb), 0, stream,
                            (const cplx<T>*)spec[0], (const cplx<T>*)spec[1],
                            (const cplx<T>*)spec[2], (const cplx<T>*)spec[3],
@@ -1450,12 +1466,6 @@ void Case<T>::advance_clocks() {
 // ---------------------------------------------------------------------------
 // Spectral-resident step (spectral.hpp)
 // ---------------------------------------------------------------------------
-template <typename T>
-static SpecGeo<T> spec_geo(const Dims& d, long msp, int k0, int nlev) {
-    return SpecGeo<T>{d.ny, d.NK, d.nz, k0, nlev, d.splane, msp, (T)(2.0 * PI_D / d.prm.lx),
-                      (T)(2.0 * PI_D / d.prm.ly)};
-}
-
 // The six stress spectra (levels 1..nz) for divstress_uv + divstress_w,
 // which k_spec_ab2 forms from them; no inverse transform.
 template <typename T>
@@ -1470,25 +1480,42 @@ void Case<T>::divstress_spec() {
     fwd2d(6, src, scs, d.plane, 1, d.field, S, d.splane, 1, msp, d.nz);
 }
 
-// press_stag_array on u*, v*, w* spectra (in sU, sV, sW; the solve scales
-// them by 1/(tadv1 dt)) and the divtz spectra of levels 1 and nz; p_hat
-// into sP.
+// The AB2 update, the pressure solve and the projection on the spectra:
+// advection in spec[0..2], stresses in spec[3..8], u, v, w in sU, sV, sW;
+// p_hat into sP.  One launch (k_column) where the grid has a plan for it, else
+// the separate kernels (k_tridag scales u*, v*, w* by 1/(tadv1 dt) and takes
+// the divtz spectra of levels 1 and nz from sDz).
 template <typename T>
-void Case<T>::press_spec() {
+void Case<T>::column_spec(const SpecAb2<T>& a) {
     TriGeo tg{d.ny, d.NK, d.nz, d.splane, msp, Ma, 2.0 * PI_D / d.prm.lx,
               2.0 * PI_D / d.prm.ly, d.dz, 1.0 / (d.dz * d.dz), 1.0 / d.dz};
     tg.hsc = (1.0 / d.tadv1) / d.prm.dt;
-    const int nsys = Ma * d.ny * d.NK;
+    const SpecGeo<T> g = spec_geo<T>(d, msp, 1, d.nz);
+    if (column_plan<T>(d.nz, d.ny * d.NK, d.splane).L) {
+        // sixteen spectra in and seven out, and the forcing on its levels
+        const double cb = (double)Ma * d.splane * sizeof(cplx<T>) *
+                          (23.0 * d.nz + (a.fx ? 3.0 * (a.kf1 - a.kf0 + 1) : 0.0));
+        timer.run(stream, KK_TRIDAG, cb, [&] {
+            launch_column<T, true>(a, ColPress<T>{}, g, tg, sP, gam, (T)d.dz, dev_err, Ma, stream);
+        });
+        return;
+    }
+    const int n = d.ny * d.NK;
+    const dim3 gs((n + BLK - 1) / BLK, d.nz * Ma);
+    hipLaunchKernelGGL(k_spec_ab2<T>, gs, dim3(BLK), 0, stream, a, g, (T)d.dz);
+    const int nsys = Ma * n, tb = choice_for<T>(PK_TRIDAG, d.ny, d.NK).S;
     const double tbytes =
         (double)Ma * d.splane * sizeof(cplx<T>) * (3.0 * d.nz + 1 + 2 + d.nz + 1);
-    const PassChoice ch = choice_for<T>(PK_TRIDAG, d.ny, d.NK);
-    const int tb = ch.S;
     timer.run(stream, KK_TRIDAG, tbytes, [&] {
         LG_LAUNCH(k_tridag<T>, dim3((nsys + tb - 1) / tb), dim3(tb), 0, stream,
                   (const cplx<T>*)sU, (const cplx<T>*)sV, (const cplx<T>*)sW,
                   (const cplx<T>*)(sDz + d.splane), (const cplx<T>*)(sDz + d.nz * d.splane),
                   sP, gam, usc, tg, dev_err);
     });
+    hipLaunchKernelGGL(k_spec_project<T>, gs, dim3(BLK), 0, stream, (const cplx<T>*)sP, sU,
+                       sV, sW, g, (T)d.prm.dt, (T)d.tadv1, (T)d.dz);
+    hipLaunchKernelGGL(k_spec_bc<T>, dim3((n + BLK - 1) / BLK, Ma), dim3(BLK), 0, stream, sU,
+                       sV, sW, g);
 }
 
 // The loop body with the state in spectra.  cold: u, v, w and RHS_f are the
@@ -1528,6 +1555,10 @@ void Case<T>::step_body_spec(bool cold) {
             hipLaunchKernelGGL(k_select_members<T>, dim3((unsigned)((n + BLK - 1) / BLK), Ma, 6),
                                dim3(BLK), 0, stream, sa, (const int*)(d_flags + 5 * M), msp, n);
         }
+        // a physical RHS_f holds its pressure gradient already
+        hipLaunchKernelGGL(k_fill_members_if<T>, dim3((unsigned)((2 * msp + BLK - 1) / BLK), Ma),
+                           dim3(BLK), 0, stream, reinterpret_cast<T*>(sPf),
+                           (const int*)(d_flags + 5 * M), 2 * msp, 2 * msp, (T)0);
     }
     filt_da_uvw(false);
     ddz_uvw();
@@ -1542,22 +1573,14 @@ void Case<T>::step_body_spec(bool cold) {
         const T scs[3] = {sc, sc, sc};
         fwd2d(3, fs, scs, d.plane, kf0, d.field, sF, d.splane, kf0, msp, kf1 - kf0 + 1);
     }
-    const int n = d.ny * d.NK;
-    const dim3 gs((n + BLK - 1) / BLK, d.nz * Ma);
-    const SpecGeo<T> g = spec_geo<T>(d, msp, 1, d.nz);
     SpecAb2<T> a{spec[0], spec[1], spec[2],
                  StressSpec<T>{spec[3], spec[4], spec[5], spec[6], spec[7], spec[8]}, sDz,
                  (T)(1.0 / d.dz),
                  tb ? sF[0] : nullptr, tb ? sF[1] : nullptr, tb ? sF[2] : nullptr,
-                 sR[0], sR[1], sR[2], sRf[0], sRf[1], sRf[2], sU, sV, sW, d_mpf,
+                 sR[0], sR[1], sR[2], sRf[0], sRf[1], sRf[2], sPf, sU, sV, sW, d_mpf,
                  (const int*)d_flags, d.prm.use_mean_p_force, kf0, kf1,
                  (T)d.prm.dt, (T)d.tadv1, (T)d.tadv2};
-    hipLaunchKernelGGL(k_spec_ab2<T>, gs, dim3(BLK), 0, stream, a, g);
-    press_spec();
-    hipLaunchKernelGGL(k_spec_project<T>, gs, dim3(BLK), 0, stream, (const cplx<T>*)sP, sR[0],
-                       sR[1], sR[2], sU, sV, sW, g, (T)d.prm.dt, (T)d.tadv1, (T)d.dz);
-    hipLaunchKernelGGL(k_spec_bc<T>, dim3((n + BLK - 1) / BLK, Ma), dim3(BLK), 0, stream, sU,
-                       sV, sW, g);
+    column_spec(a);
 }
 
 // The storage exchange of a step (RHS_f = RHS): physical and spectral RHS,
@@ -1571,6 +1594,7 @@ void Case<T>::swap_rhs() {
     swapped = !swapped;
     if (!spec_on) return;
     for (int q = 0; q < 3; ++q) std::swap(sR[q], sRf[q]);
+    std::swap(sP, sPf);
     std::swap(fld[LG_FXA], fprev[0]);
     std::swap(fld[LG_FYA], fprev[1]);
     std::swap(fld[LG_FZA], fprev[2]);
@@ -1651,6 +1675,15 @@ void Case<T>::rhs_high(T* const* f, T* const* t, T* const* g, T* const* scratch)
                        (const T*)scratch[2], f != nullptr, GEO(1, n1), (T)(1.0 / d.dz));
 }
 
+// The reference's RHS (or RHS_f) spectra, R - grad p, into spec[0..2].
+template <typename T>
+void Case<T>::spec_rhs(cplx<T>* const* r, const cplx<T>* p) {
+    const int n = d.ny * d.NK;
+    hipLaunchKernelGGL(k_spec_rhs<T>, dim3((n + BLK - 1) / BLK, d.nz * Ma), dim3(BLK), 0, stream,
+                       (const cplx<T>*)r[0], (const cplx<T>*)r[1], (const cplx<T>*)r[2], p,
+                       spec[0], spec[1], spec[2], spec_geo<T>(d, msp, 1, d.nz), (T)d.dz);
+}
+
 // Make the stale physical fields of `groups` from the spectra, with the
 // high-wavenumber remainders (rhs_high) added back where the reference's
 // fields hold them.
@@ -1727,7 +1760,8 @@ void Case<T>::materialize(unsigned groups) {
                      {LG_W, 0, BOGUS}});
     }
     if (groups & SG_RHS) {
-        const cplx<T>* is[3] = {sR[0], sR[1], sR[2]};
+        const cplx<T>* is[3] = {spec[0], spec[1], spec[2]};
+        spec_rhs(sR, sP);
         T* dst[3] = {fld[LG_RHSX], fld[LG_RHSY], fld[LG_RHSZ]};
         inv2d(3, is, on, d.splane, 1, msp, dst, d.plane, 1, d.field, nz, tsp);
         for (int q = 0; q < 3; ++q)
@@ -1740,7 +1774,8 @@ void Case<T>::materialize(unsigned groups) {
         // RHS_f = the previous RHS (or the physical input of a step that
         // started from it), or this step's (before - grad p) for an Euler
         // member
-        const cplx<T>* is[3] = {sRf[0], sRf[1], sRf[2]};
+        const cplx<T>* is[3] = {spec[0], spec[1], spec[2]};
+        spec_rhs(sRf, sPf);
         T* dst[3] = {fld[LG_RHSX_F], fld[LG_RHSY_F], fld[LG_RHSZ_F]};
         inv2d(3, is, on, d.splane, 1, msp, dst, d.plane, 1, d.field, nz, tsp);
         for (int q = 0; q < 3; ++q)
@@ -1796,7 +1831,7 @@ int Case<T>::count_cold() const {
 template <typename T>
 void Case<T>::copy_spec_member(int src, int dst) {
     if (!spec_on) return;
-    cplx<T>* bufs[10] = {sU, sV, sW, sR[0], sR[1], sR[2], sRf[0], sRf[1], sRf[2], sP};
+    cplx<T>* bufs[11] = {sU, sV, sW, sR[0], sR[1], sR[2], sRf[0], sRf[1], sRf[2], sP, sPf};
     for (cplx<T>* b : bufs)
         LG_HIP(hipMemcpyAsync(b + (long)dst * msp, b + (long)src * msp, msp * sizeof(cplx<T>),
                               hipMemcpyDeviceToDevice, stream));

@@ -76,6 +76,9 @@ struct TurbineSet {
     ~TurbineSet();
 };
 
+template <typename T>
+struct SpecAb2;
+
 // Batch of M same-grid members.  Member m of every array starts at
 // m * (its member stride); Ma <= M members are stepped.
 template <typename T>
@@ -142,9 +145,10 @@ struct Case {
     // before a disk-set change becomes the write target and is cleared
     int fclear_pending = 0;
     unsigned stale = 0;
-    cplx<T>* sR[3] = {};             // RHS spectra (after - grad p)
-    cplx<T>* sRf[3] = {};            // RHS_f spectra
-    cplx<T>* sP = nullptr;           // pressure spectrum, levels 0..nz
+    cplx<T>* sR[3] = {};             // RHS spectra before - grad p
+    cplx<T>* sRf[3] = {};            // RHS_f spectra, alike
+    cplx<T>* sP = nullptr;           // pressure spectrum of RHS's step, levels 0..nz
+    cplx<T>* sPf = nullptr;          // of RHS_f's (zero where RHS_f holds - grad p already)
     cplx<T>* sDz = nullptr;          // divtz spectra of the step (levels 1 and nz only)
     cplx<T>* sF[3] = {};             // forcing spectra of the step (disk levels)
     T* fprev[3] = {};                // the previous step's fxa, fya, fza
@@ -165,6 +169,7 @@ struct Case {
     T* fld[LG_NFIELDS] = {};
     // spectral scratch, each (nz+1) small spectral planes
     static constexpr int NSPEC = 12;
+    cplx<T>* spool = nullptr;        // every spectrum of the case (spec, sU ... sDz)
     cplx<T>* spec[NSPEC] = {};
     // big-grid scratch (levels 0..nz)
     static constexpr int NBIG = 9;
@@ -260,10 +265,11 @@ struct Case {
     void run_body(bool cold);
     void after_body();
     void divstress_spec();
-    void press_spec();
+    void column_spec(const SpecAb2<T>& a);
     void materialize(unsigned groups);
     void touch(bool modify);
     void high_part(T* const* f, T* const* out, int nf, int ka, int kb);
+    void spec_rhs(cplx<T>* const* r, const cplx<T>* p);
     void rhs_high(T* const* f, T* const* t, T* const* g, T* const* scratch);
     void step();
     void step_graph();

@@ -56,8 +56,48 @@ __device__ __forceinline__ void spec_k(const SpecGeo<T>& g, int j, int c, T& kx,
     ky = g.kys * (T)my;
 }
 
+// The step's spectral arithmetic with its roundings fixed (the fused
+// multiply-adds written out), so that every kernel that forms a quantity
+// forms the same bits: the stress divergence i kx A + i ky B, RHS - i k p,
+// u + dt (t1 R + t2 F) and u - dt t1 i k p.
+__device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 template <typename T>
-__device__ __forceinline__ cplx<T> cik(cplx<T> v, T k) { return cplx<T>{-v.y * k, v.x * k}; }
+__device__ __forceinline__ cplx<T> div_ik(cplx<T> a, cplx<T> b, T kx, T ky) {
+#pragma clang fp contract(off)
+    return cplx<T>{fma_t(ky, -b.y, -(kx * a.y)), fma_t(ky, b.x, kx * a.x)};
+}
+template <typename T>
+__device__ __forceinline__ cplx<T> add_dz(cplx<T> a, cplx<T> hi, cplx<T> lo, T rdz) {
+#pragma clang fp contract(off)
+    return cplx<T>{fma_t(rdz, hi.x - lo.x, a.x), fma_t(rdz, hi.y - lo.y, a.y)};
+}
+template <typename T>
+__device__ __forceinline__ cplx<T> sub_ik(cplx<T> r, cplx<T> p, T k) {
+    return cplx<T>{fma_t(k, p.y, r.x), fma_t(-p.x, k, r.y)};
+}
+template <typename T>
+__device__ __forceinline__ cplx<T> ab2_of(cplx<T> u, cplx<T> R, cplx<T> F, T dt, T t1, T t2) {
+#pragma clang fp contract(off)
+    return cplx<T>{fma_t(dt, fma_t(t1, R.x, t2 * F.x), u.x),
+                   fma_t(dt, fma_t(t1, R.y, t2 * F.y), u.y)};
+}
+template <typename T>
+__device__ __forceinline__ cplx<T> proj_ik(cplx<T> u, cplx<T> p, T k, T dt, T t1) {
+#pragma clang fp contract(off)
+    return cplx<T>{fma_t(dt, t1 * (k * p.y), u.x), fma_t(-dt, t1 * (p.x * k), u.y)};
+}
+// d p / dz from level k - 1 to k, and u - dt t1 of it
+template <typename T>
+__device__ __forceinline__ cplx<T> dz_p(cplx<T> pk, cplx<T> pm, T dzv) {
+    return cplx<T>{(pk.x - pm.x) / dzv, (pk.y - pm.y) / dzv};
+}
+template <typename T>
+__device__ __forceinline__ cplx<T> proj_dz(cplx<T> u, cplx<T> gz, T dt, T t1) {
+#pragma clang fp contract(off)
+    return cplx<T>{fma_t(-dt, t1 * gz.x, u.x), fma_t(-dt, t1 * gz.y, u.y)};
+}
 
 // Divergence of the stresses from their spectra (divstress_uv.f90:21-85,
 // divstress_w.f90:21-116) at mode o of level k: divtx, divty on 1..nz-1
@@ -73,29 +113,27 @@ __device__ __forceinline__ cplx<T> divt_xy(const cplx<T>* a, const cplx<T>* b, c
                                            long o, long S, bool nyq, T kx, T ky, T rdz) {
     const cplx<T> p = a[o], q = b[o];
     const cplx<T> z1 = zt[o + S], z0 = zt[o];
-    const cplx<T> dxy = nyq ? cplx<T>{(T)0, (T)0}
-                            : cplx<T>{-p.y * kx + -q.y * ky, p.x * kx + q.x * ky};
-    return cplx<T>{dxy.x + rdz * (z1.x - z0.x), dxy.y + rdz * (z1.y - z0.y)};
+    const cplx<T> dxy = nyq ? cplx<T>{(T)0, (T)0} : div_ik(p, q, kx, ky);
+    return add_dz(dxy, z1, z0, rdz);
 }
 
 template <typename T>
 __device__ __forceinline__ cplx<T> divt_z(const StressSpec<T>& t, long o, long S, int k, int nz,
                                           bool nyq, T kx, T ky, T rdz) {
     const cplx<T> p = t.txz[o], q = t.tyz[o];
-    cplx<T> z = nyq ? cplx<T>{(T)0, (T)0}
-                    : cplx<T>{-p.y * kx + -q.y * ky, p.x * kx + q.x * ky};
-    if (k >= 2 && k <= nz - 1) {
-        const cplx<T> z1 = t.tzz[o], z0 = t.tzz[o - S];
-        z = cplx<T>{z.x + rdz * (z1.x - z0.x), z.y + rdz * (z1.y - z0.y)};
-    }
-    return z;
+    const cplx<T> z = nyq ? cplx<T>{(T)0, (T)0} : div_ik(p, q, kx, ky);
+    return k >= 2 && k <= nz - 1 ? add_dz(z, t.tzz[o], t.tzz[o - S], rdz) : z;
 }
 
 // RHS assembly and AB2 update (main.f90:211-296) on the spectra, levels
 // 1..nz: R = -conv - divt (+ mean pressure force on the (0,0) mode)
 // (+ the disks' forcing on levels kf0..kf1) for x, y on 1..nz-1 and z on
-// 1..nz (no forcing at nz); members with euler[m] take R_f = R; then
-// u* = u + dt (t1 R + t2 R_f) in place of u (x, y on 1..nz-1, z on 1..nz).
+// 1..nz (no forcing at nz).  The stored spectra of RHS and RHS_f are R
+// without its step's pressure gradient, kept beside that step's p_hat: the
+// reference's RHS -= grad p (main.f90:321-326) is applied where they are
+// read (sub_ik, dz_p; 3 spectra less read and written a step).  So
+// u* = u + dt (t1 R + t2 (R_f - grad p_f)) in place of u (x, y on 1..nz-1,
+// z on 1..nz); members with euler[m] take R_f = R, p_f = 0.
 // divt is formed here from the stress spectra; its z component at levels 1
 // and nz (the pressure solve's boundary rows) is also stored in dvz_bc.
 template <typename T>
@@ -107,6 +145,7 @@ struct SpecAb2 {
     const cplx<T> *fx, *fy, *fz;       // forcing spectra (levels kf0..kf1) or null
     cplx<T> *rx, *ry, *rz;             // R out
     cplx<T> *rfx, *rfy, *rfz;          // R_f in (out for Euler members)
+    cplx<T>* pf;                       // its step's p_hat, levels 0..nz (alike)
     cplx<T> *ux, *uy, *uz;             // u in, u* out
     const double* mpf;                 // 2 per member
     const int* euler;
@@ -115,7 +154,7 @@ struct SpecAb2 {
 };
 
 template <typename T>
-__global__ void k_spec_ab2(SpecAb2<T> a, SpecGeo<T> g) {
+__global__ void k_spec_ab2(SpecAb2<T> a, SpecGeo<T> g, T dzv) {
     int m, k, j, c;
     long o;
     if (!spec_of(g, m, k, j, c, o)) return;
@@ -126,8 +165,13 @@ __global__ void k_spec_ab2(SpecAb2<T> a, SpecGeo<T> g) {
     spec_k(g, j, c, kx, ky);
     const bool nyq = j == g.ny / 2;
     const long S = g.splane;
+    cplx<T> pk{}, gz{};
+    if (!eu) {
+        pk = a.pf[o];
+        gz = dz_p(pk, a.pf[o - S], dzv);
+    }
     auto upd = [&](const cplx<T>* cv, const cplx<T> dd, const cplx<T>* fv, cplx<T>* r,
-                   cplx<T>* rf, cplx<T>* u, T mp, bool mpf_on) {
+                   cplx<T>* rf, int q, cplx<T>* u, T mp, bool mpf_on) {
         const cplx<T> cc = cv[o];
         cplx<T> R{-cc.x - dd.x, -cc.y - dd.y};
         if (mpf_on && zero_mode) R.x = R.x + mp;
@@ -138,57 +182,62 @@ __global__ void k_spec_ab2(SpecAb2<T> a, SpecGeo<T> g) {
         r[o] = R;
         cplx<T> F = R;
         if (eu) rf[o] = R;
-        else F = rf[o];
-        const cplx<T> uu = u[o];
-        u[o] = cplx<T>{uu.x + a.dt * (a.t1 * R.x + a.t2 * F.x),
-                       uu.y + a.dt * (a.t1 * R.y + a.t2 * F.y)};
+        else F = q == 2 ? csub(rf[o], gz) : sub_ik(rf[o], pk, q ? ky : kx);
+        u[o] = ab2_of(u[o], R, F, a.dt, a.t1, a.t2);
     };
     if (k <= g.nz - 1) {
         const cplx<T> dvx = divt_xy(a.ts.txx, a.ts.txy, a.ts.txz, o, S, nyq, kx, ky, a.rdz);
         const cplx<T> dvy = divt_xy(a.ts.txy, a.ts.tyy, a.ts.tyz, o, S, nyq, kx, ky, a.rdz);
-        upd(a.cx, dvx, forced ? a.fx : nullptr, a.rx, a.rfx, a.ux, (T)a.mpf[2 * m],
+        upd(a.cx, dvx, forced ? a.fx : nullptr, a.rx, a.rfx, 0, a.ux, (T)a.mpf[2 * m],
             a.use_mpf != 0);
-        upd(a.cy, dvy, forced ? a.fy : nullptr, a.ry, a.rfy, a.uy, (T)a.mpf[2 * m + 1],
+        upd(a.cy, dvy, forced ? a.fy : nullptr, a.ry, a.rfy, 1, a.uy, (T)a.mpf[2 * m + 1],
             a.use_mpf != 0);
     }
     const cplx<T> dvz = divt_z(a.ts, o, S, k, g.nz, nyq, kx, ky, a.rdz);
     if (k == 1 || k == g.nz) a.dvz_bc[o] = dvz;
-    upd(a.cz, dvz, forced ? a.fz : nullptr, a.rz, a.rfz, a.uz, (T)0, false);
+    upd(a.cz, dvz, forced ? a.fz : nullptr, a.rz, a.rfz, 2, a.uz, (T)0, false);
+    if (eu) {
+        a.pf[o] = cplx<T>{(T)0, (T)0};
+        if (k == 1) a.pf[o - S] = cplx<T>{(T)0, (T)0};
+    }
 }
 
-// RHS -= grad p and the projection (main.f90:321-326, forcing.f90:149-244)
-// on the spectra, levels 1..nz: dpdx, dpdy = i kx p, i ky p (1..nz-1);
-// dpdz = (p(k) - p(k-1)) / dz (1..nz); u = u* - dt t1 dpdx (1..nz-1),
-// w = w* - dt t1 dpdz (2..nz-1).  The lid and wall rows follow in
+// The projection (forcing.f90:149-244) on the spectra: dpdx, dpdy = i kx p,
+// i ky p (1..nz-1); dpdz = (p(k) - p(k-1)) / dz; u = u* - dt t1 dpdx
+// (1..nz-1), w = w* - dt t1 dpdz (2..nz-1).  The lid and wall rows follow in
 // k_spec_bc.
 template <typename T>
-__global__ void k_spec_project(const cplx<T>* p, cplx<T>* rx, cplx<T>* ry, cplx<T>* rz,
-                               cplx<T>* ux, cplx<T>* uy, cplx<T>* uz, SpecGeo<T> g, T dt, T t1,
-                               T dzv) {
+__global__ void k_spec_project(const cplx<T>* p, cplx<T>* ux, cplx<T>* uy, cplx<T>* uz,
+                               SpecGeo<T> g, T dt, T t1, T dzv) {
+    int m, k, j, c;
+    long o;
+    if (!spec_of(g, m, k, j, c, o)) return;
+    if (k > g.nz - 1) return;
+    T kx, ky;
+    spec_k(g, j, c, kx, ky);
+    const cplx<T> pk = p[o];
+    ux[o] = proj_ik(ux[o], pk, kx, dt, t1);
+    uy[o] = proj_ik(uy[o], pk, ky, dt, t1);
+    if (k >= 2) uz[o] = proj_dz(uz[o], dz_p(pk, p[o - g.splane], dzv), dt, t1);
+}
+
+// The reference's RHS (or RHS_f) spectra: R - grad p (main.f90:321-326),
+// levels 1..nz (x, y: 1..nz-1).
+template <typename T>
+__global__ void k_spec_rhs(const cplx<T>* rx, const cplx<T>* ry, const cplx<T>* rz,
+                           const cplx<T>* p, cplx<T>* ox, cplx<T>* oy, cplx<T>* oz, SpecGeo<T> g,
+                           T dzv) {
     int m, k, j, c;
     long o;
     if (!spec_of(g, m, k, j, c, o)) return;
     T kx, ky;
     spec_k(g, j, c, kx, ky);
-    const cplx<T> pk = p[o], pm = p[o - g.splane];
-    const cplx<T> gz{(pk.x - pm.x) / dzv, (pk.y - pm.y) / dzv};
+    const cplx<T> pk = p[o];
     if (k <= g.nz - 1) {
-        const cplx<T> gx = cik(pk, kx), gy = cik(pk, ky);
-        cplx<T> r = rx[o];
-        rx[o] = cplx<T>{r.x - gx.x, r.y - gx.y};
-        r = ry[o];
-        ry[o] = cplx<T>{r.x - gy.x, r.y - gy.y};
-        cplx<T> u = ux[o];
-        ux[o] = cplx<T>{u.x + dt * (-(t1 * gx.x)), u.y + dt * (-(t1 * gx.y))};
-        u = uy[o];
-        uy[o] = cplx<T>{u.x + dt * (-(t1 * gy.x)), u.y + dt * (-(t1 * gy.y))};
+        ox[o] = sub_ik(rx[o], pk, kx);
+        oy[o] = sub_ik(ry[o], pk, ky);
     }
-    cplx<T> r = rz[o];
-    rz[o] = cplx<T>{r.x - gz.x, r.y - gz.y};
-    if (k >= 2 && k <= g.nz - 1) {
-        const cplx<T> u = uz[o];
-        uz[o] = cplx<T>{u.x + dt * (-(t1 * gz.x)), u.y + dt * (-(t1 * gz.y))};
-    }
+    oz[o] = csub(rz[o], dz_p(pk, p[o - g.splane], dzv));
 }
 
 // Boundary rows of the projected velocity (forcing.f90:226-243, main.f90:

@@ -35,7 +35,7 @@ enum KernelKind : int {
     KK_ROWS_C2R = 1,          // inverse rows, nx points
     KK_COLS_FWD = 2,          // forward columns, ny points
     KK_COLS_INV = 3,          // inverse columns, ny points
-    KK_TRIDAG = 4,            // pressure tridiagonal
+    KK_TRIDAG = 4,            // pressure solve (spectral step: the whole column pass)
     KK_ROWS_R2C_PAD = 5,      // forward rows on the 3/2 grid
     KK_ROWS_C2R_PAD = 6,      // inverse rows on the 3/2 grid
     KK_COLS_UNPAD = 7,        // forward columns 3/2 grid -> small
