@@ -833,9 +833,51 @@ void Case<T>::ddz_uvw() {
                            fld[LG_DUDZ], fld[LG_DVDZ], fld[LG_DWDZ], GEO(1, nch),
                            (T)(1.0 / d.dz));
     }
-    fill_levels({{LG_DUDZ, 0, BOGUS}, {LG_DUDZ, 1, BOGUS}, {LG_DUDZ, d.nz, BOGUS},
-                 {LG_DVDZ, 0, BOGUS}, {LG_DVDZ, 1, BOGUS}, {LG_DVDZ, d.nz, BOGUS},
-                 {LG_DWDZ, 0, BOGUS}, {LG_DWDZ, d.nz, BOGUS}});
+}
+
+// The planes whose values a step does not compute: BOGUS at the ghost level
+// and where the reference leaves it (derivatives.f90:214-311,
+// sgs_stag_util.f90:33-464), the lid's stresses and derivatives zero
+// (wallstress.f90:21-257, ubc_mom = 0).  Nothing but the host writes them, so a
+// spectral-resident case sets them on the steps that start from physical
+// fields only, in both buffers of the exchanged stresses and for every
+// member; the all-physical step at its head (one launch a step instead of
+// three: 32^3 FP64 2.6 us a launch, 256 x 256 x 192 4.8 us).
+template <typename T>
+void Case<T>::fill_const_planes() {
+    const int nz = d.nz;
+    FillList<T> a{};
+    int n = 0;
+    auto put = [&](T* f, int k, double v) {
+        a.p[n] = f + (long)k * d.plane;
+        a.v[n++] = (T)v;
+    };
+    for (int id : {LG_DUDZ, LG_DVDZ}) {
+        put(fld[id], 0, BOGUS);
+        put(fld[id], 1, BOGUS);
+        put(fld[id], nz, 0.0);
+    }
+    put(fld[LG_DWDZ], 0, BOGUS);
+    put(fld[LG_DWDZ], nz, BOGUS);
+    for (int id : {LG_TXX, LG_TXY, LG_TYY, LG_TZZ}) {
+        put(fld[id], 0, BOGUS);
+        put(fld[id], nz, BOGUS);
+    }
+    for (int id : {LG_TXZ, LG_TYZ}) {
+        put(fld[id], 0, BOGUS);
+        put(fld[id], nz, 0.0);
+    }
+    if (spec_on) {
+        for (int q = 0; q < 3; ++q) {
+            put(tprev[q], 0, BOGUS);
+            put(tprev[q], nz, q < 2 ? 0.0 : BOGUS);
+        }
+    }
+    static_assert(26 <= MAX_FILLS, "fill_const_planes needs more entries");
+    a.mstride = d.field;
+    a.plane = d.plane;
+    hipLaunchKernelGGL(k_fill_list<T>, dim3((unsigned)((d.plane + BLK - 1) / BLK), M, n),
+                       dim3(BLK), 0, stream, a);
 }
 
 // One plane per member (member stride = field) filtered by op.
@@ -861,7 +903,7 @@ void Case<T>::test_filter_plane(const T* in, T* out, int op) {
 // outside it and on the Nyquist row; the band mask also drops the kx Nyquist
 // column, which the physical u, v do not carry).
 template <typename T>
-void Case<T>::wallstress(const cplx<T>* su, const cplx<T>* sv) {
+void Case<T>::wallstress(const cplx<T>* su, const cplx<T>* sv, bool fill) {
     const T one = (T)1;
     const cplx<T>* s2[2] = {spec[4], spec[5]};
     int ops[2] = {OP_G1, OP_G1};
@@ -882,8 +924,9 @@ void Case<T>::wallstress(const cplx<T>* su, const cplx<T>* sv) {
                        (const T*)tmp[0], (const T*)tmp[1], d.field, (const T*)fld[LG_U],
                        (const T*)fld[LG_V], fld[LG_TXZ], fld[LG_TYZ], fld[LG_DUDZ], fld[LG_DVDZ],
                        GEO(1, 1), (const double*)d_denom, d.prm.vonk, d.dz);
-    fill_levels({{LG_TXZ, d.nz, 0.0}, {LG_TYZ, d.nz, 0.0}, {LG_DUDZ, d.nz, 0.0},
-                 {LG_DVDZ, d.nz, 0.0}});
+    if (fill)
+        fill_levels({{LG_TXZ, d.nz, 0.0}, {LG_TYZ, d.nz, 0.0}, {LG_DUDZ, d.nz, 0.0},
+                     {LG_DVDZ, d.nz, 0.0}});
 }
 
 // ---------------------------------------------------------------------------
@@ -899,7 +942,7 @@ void Case<T>::calc_sij() {
 }
 
 template <typename T>
-void Case<T>::sgs_stag() {
+void Case<T>::sgs_stag(bool fill) {
     // without a dynamic-model update between them, S_ij and the stresses
     // are formed in one pass (k_sij_tau); Cs_opt2 is set first either way
     if (lag_now) calc_sij();
@@ -932,9 +975,11 @@ void Case<T>::sgs_stag() {
         if (lag_now) stale &= ~(unsigned)SG_SIJ;
         else stale |= SG_SIJ;
     }
-    fill_levels({{LG_TXX, 0, BOGUS}, {LG_TXY, 0, BOGUS}, {LG_TXZ, 0, BOGUS}, {LG_TYY, 0, BOGUS},
-                 {LG_TYZ, 0, BOGUS}, {LG_TZZ, 0, BOGUS}, {LG_TXX, d.nz, BOGUS},
-                 {LG_TXY, d.nz, BOGUS}, {LG_TYY, d.nz, BOGUS}, {LG_TZZ, d.nz, BOGUS}});
+    if (fill)
+        fill_levels({{LG_TXX, 0, BOGUS}, {LG_TXY, 0, BOGUS}, {LG_TXZ, 0, BOGUS},
+                     {LG_TYY, 0, BOGUS}, {LG_TYZ, 0, BOGUS}, {LG_TZZ, 0, BOGUS},
+                     {LG_TXX, d.nz, BOGUS}, {LG_TXY, d.nz, BOGUS}, {LG_TYY, d.nz, BOGUS},
+                     {LG_TZZ, d.nz, BOGUS}});
 }
 
 // ---------------------------------------------------------------------------
@@ -1381,10 +1426,11 @@ void Case<T>::rhs_gradp() {
 template <typename T>
 void Case<T>::step_body() {
     clock_begin();
+    fill_const_planes();
     filt_da_uvw();
     ddz_uvw();
-    wallstress();
-    sgs_stag();
+    wallstress(nullptr, nullptr, false);
+    sgs_stag(false);
     divstress_uvw();
     convec(true);
     if (turb) turbines_forcing();
@@ -1525,6 +1571,7 @@ template <typename T>
 void Case<T>::step_body_spec(bool cold) {
     const T sc = (T)(1.0 / (d.nx * d.ny));
     if (cold) {
+        fill_const_planes();
         // spectra of the cold members' physical u, v, w (levels 0..nz) and
         // RHS_f (x, y on 1..nz-1, z on 1..nz): straight into the state when
         // every member is cold, else into scratch and then per member
@@ -1562,8 +1609,8 @@ void Case<T>::step_body_spec(bool cold) {
     }
     filt_da_uvw(false);
     ddz_uvw();
-    wallstress(sU, sV);
-    sgs_stag();
+    wallstress(sU, sV, false);
+    sgs_stag(false);
     convec(true, true);
     divstress_spec();
     const bool tb = turb && turb->total_nodes > 0 && kf1 >= kf0;

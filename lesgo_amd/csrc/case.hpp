@@ -234,9 +234,11 @@ struct Case {
     void ddz_w(int f, int dfdz);
     void ddz_uvw();        // ddz_uv(u), ddz_uv(v), ddz_w(w): one pass, the same values
     void test_filter_plane(const T* in, T* out, int op);
-    void wallstress(const cplx<T>* su = nullptr, const cplx<T>* sv = nullptr);
+    void fill_const_planes();
+    // fill: set the lid's (ghost) planes too (a step has set them already)
+    void wallstress(const cplx<T>* su = nullptr, const cplx<T>* sv = nullptr, bool fill = true);
     void calc_sij();
-    void sgs_stag();
+    void sgs_stag(bool fill = true);
     void interpolag_sdep(bool in_place = true);
     void lagrange_sdep();
     void divstress_uv();

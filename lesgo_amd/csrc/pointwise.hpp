@@ -41,9 +41,9 @@ __global__ void k_fill_planes(T* f, long mstride, long n, T v) {
     if (idx < n) f[(long)blockIdx.y * mstride + idx] = v;
 }
 
-// Up to 16 (plane, value) fills in one launch: grid (blocks per plane,
+// Up to MAX_FILLS (plane, value) fills in one launch: grid (blocks per plane,
 // members, entries); entry q sets p[q][m * mstride + i] = v[q], i < plane.
-constexpr int MAX_FILLS = 16;
+constexpr int MAX_FILLS = 32;
 template <typename T>
 struct FillList {
     T* p[MAX_FILLS];
