@@ -942,7 +942,7 @@ void Case<T>::calc_sij() {
 }
 
 template <typename T>
-void Case<T>::sgs_stag(bool fill) {
+void Case<T>::sgs_stag(bool fill, bool from_uvw) {
     // without a dynamic-model update between them, S_ij and the stresses
     // are formed in one pass (k_sij_tau); Cs_opt2 is set first either way
     if (lag_now) calc_sij();
@@ -967,8 +967,13 @@ void Case<T>::sgs_stag(bool fill) {
                       fld[LG_S12], fld[LG_S13], fld[LG_S22], fld[LG_S23], fld[LG_S33]};
         // a spectral-resident case leaves S_ij and Nu_t to be made on demand
         const int nch = (d.nz + SIJ_L - 1) / SIJ_L;
-        hipLaunchKernelGGL(k_sij_tau<T>, grid_ij(d.nx, d.ny, nch, Ma), dim3(BLK), 0, stream,
-                           sa, a, GEO(1, d.nz), spec_on ? 0 : 1);
+        if (from_uvw)
+            hipLaunchKernelGGL(k_sij_tau_uvw<T>, grid_ij(d.nx, d.ny, nch, Ma), dim3(BLK), 0,
+                               stream, sa, a, (const T*)fld[LG_U], (const T*)fld[LG_V],
+                               (const T*)fld[LG_W], (T)(1.0 / d.dz), GEO(1, d.nz));
+        else
+            hipLaunchKernelGGL(k_sij_tau<T>, grid_ij(d.nx, d.ny, nch, Ma), dim3(BLK), 0, stream,
+                               sa, a, GEO(1, d.nz), spec_on ? 0 : 1);
     }
     if (spec_on) {
         // (after_body does the same for whole steps, replayed graphs included)
@@ -1608,9 +1613,10 @@ void Case<T>::step_body_spec(bool cold) {
                            (const int*)(d_flags + 5 * M), 2 * msp, 2 * msp, (T)0);
     }
     filt_da_uvw(false);
-    ddz_uvw();
+    // the stress pass forms d/dz of u, v, w itself; the dynamic model reads them
+    if (lag_now) ddz_uvw();
     wallstress(sU, sV, false);
-    sgs_stag(false);
+    sgs_stag(false, true);
     convec(true, true);
     divstress_spec();
     const bool tb = turb && turb->total_nodes > 0 && kf1 >= kf0;
@@ -1679,8 +1685,9 @@ void Case<T>::after_body() {
         if (cold && any_euler) stale |= SG_RHSF;
         // S_ij and Nu_t are stored only by a step with a dynamic-model update
         // (set here too: a replayed graph runs no host code of sgs_stag)
-        if (lag_now) stale &= ~(unsigned)SG_SIJ;
-        else stale |= SG_SIJ;
+        // (nor the z derivatives)
+        if (lag_now) stale &= ~(unsigned)(SG_SIJ | SG_DDZ);
+        else stale |= SG_SIJ | SG_DDZ;
         std::fill(mcold.begin(), mcold.end(), 0);
     }
     if (st.on) stats_after_step();
@@ -1738,6 +1745,10 @@ template <typename T>
 void Case<T>::materialize(unsigned groups) {
     groups &= stale;
     if (!groups) return;
+    // the z derivatives are those of the step's u, v, w, which the fields
+    // hold until the end-of-step velocity replaces them; S_ij takes them
+    if (groups & (SG_UVW | SG_SIJ)) groups |= stale & SG_DDZ;
+    if (groups & SG_DDZ) ddz_uvw();
     const int nz = d.nz, n1 = nz - 1;
     // gc: this step's remainder; gq: the previous step's (or the high part of
     // a physical RHS_f); hs: scratch of rhs_high
@@ -1966,6 +1977,7 @@ void Case<T>::step_graph() {
 // ---------------------------------------------------------------------------
 template <typename T>
 double Case<T>::rmsdiv(int m) {
+    materialize(SG_DDZ);
     const int nb = 256;
     hipLaunchKernelGGL(k_rmsdiv_part<T>, dim3(nb), dim3(BLK), 0, stream,
                        (const T*)mem(LG_DUDX, m), (const T*)mem(LG_DVDY, m),

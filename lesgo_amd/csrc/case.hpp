@@ -120,9 +120,11 @@ struct Case {
     // describe it); stale: the physical groups not yet made.
     // SG_SIJ: S_ij and Nu_t, which a step without a dynamic-model update
     // does not store (only the host reads them then; made from the
-    // derivative fields, which stay valid until the next step)
+    // derivative fields, which stay valid until the next step);
+    // SG_DDZ: dudz, dvdz, dwdz, likewise
     enum : unsigned {
-        SG_UVW = 1, SG_RHS = 2, SG_RHSF = 4, SG_P = 8, SG_DIVT = 16, SG_SIJ = 32, SG_ALL = 63
+        SG_UVW = 1, SG_RHS = 2, SG_RHSF = 4, SG_P = 8, SG_DIVT = 16, SG_SIJ = 32, SG_DDZ = 64,
+        SG_ALL = 127
     };
     bool spec_on = false;
     // the Lagrangian model's inverse row pass forms the tensor contractions
@@ -238,7 +240,8 @@ struct Case {
     // fill: set the lid's (ghost) planes too (a step has set them already)
     void wallstress(const cplx<T>* su = nullptr, const cplx<T>* sv = nullptr, bool fill = true);
     void calc_sij();
-    void sgs_stag(bool fill = true);
+    // from_uvw: without a dynamic-model update, form d/dz of u, v, w in the pass
+    void sgs_stag(bool fill = true, bool from_uvw = false);
     void interpolag_sdep(bool in_place = true);
     void lagrange_sdep();
     void divstress_uv();

@@ -499,6 +499,130 @@ __global__ void k_sij_tau(SijArgs<T> sa, TauArgs<T> a, Geo g, int store_s) {
     }
 }
 
+// k_sij_tau for the spectral-resident step: the stresses alone, with the z
+// derivatives formed here from u, v, w (ddz_uv, ddz_w, derivatives.f90:214-311:
+// k_ddz_uvw's expressions, so the same bits) instead of read: u, v, w take the
+// place of dudz, dvdz, dwdz in the loads, and the pass that wrote those three
+// (256 x 256 x 192: 64 us FP32, 120 us FP64) runs only when the host reads them
+// or the dynamic model does.  dudz, dvdz come from their planes at the wall
+// (the wall model's) and are zero at the lid.
+//
+// Bound by HBM: ten fields in, six out.  One thread per (i, j) and chunk of
+// SIJ_L levels, marching up; level k + 2 (its w: k + 3) is loaded before level
+// k's stores.
+template <typename T>
+struct Raw9 {
+    T ux, uy, vx, vy, wx, wy, u, v, w;
+};
+
+template <typename T>
+__global__ void k_sij_tau_uvw(SijArgs<T> sa, TauArgs<T> a, const T* u, const T* v, const T* w,
+                              T rdz, Geo g) {
+    // no FMA contraction: as in k_sij_tau and k_ddz_uvw
+#pragma clang fp contract(off)
+    int j, i;
+    if (!ij_of(g.nx, g.ny, j, i)) return;
+    const int nz = g.nz;
+    const int nch = (nz + SIJ_L - 1) / SIJ_L;
+    const int m = blockIdx.y / nch;
+    const int kb = 1 + (int)(blockIdx.y - m * nch) * SIJ_L;
+    const int ke = min(kb + SIJ_L - 1, nz);
+    const long P = g.plane;
+    const long base = (long)m * g.mstride + (long)j * g.ld + i;
+    const T nu = a.nu;
+    // everything but w at level k
+    auto raw = [&](int k) {
+        const long o = base + (long)k * P;
+        return Raw9<T>{sa.dudx[o], sa.dudy[o], sa.dvdx[o], sa.dvdy[o],
+                       sa.dwdx[o], sa.dwdy[o], u[o],       v[o],       (T)0};
+    };
+    auto w_at = [&](int k) { return w[base + (long)k * P]; };
+    // the nine derivatives at level k >= 2 (uz, vz from the level below; wz not
+    // used at the lid)
+    auto der = [&](const Raw9<T>& r, const Raw9<T>& below, T w_up, int k) {
+        const T uz = k == nz ? (T)0 : rdz * (r.u - below.u);
+        const T vz = k == nz ? (T)0 : rdz * (r.v - below.v);
+        return Der9<T>{r.ux, r.uy, uz, r.vx, r.vy, vz, r.wx, r.wy, rdz * (w_up - r.w)};
+    };
+    Raw9<T> r0 = raw(kb), r1{};
+    r0.w = w_at(kb);
+    const int k1 = min(kb + 1, nz);
+    r1 = raw(k1);
+    r1.w = w_at(k1);
+    T w2 = w_at(min(kb + 2, nz));
+    Der9<T> d, dm{};
+    if (kb == 1) {
+        const long o = base + P;
+        d = Der9<T>{r0.ux, r0.uy, sa.dudz[o], r0.vx, r0.vy, sa.dvdz[o], r0.wx, r0.wy,
+                    rdz * (r1.w - r0.w)};
+    } else {
+        // (S_ij at kb takes no z derivative of u, v from the level below)
+        const Raw9<T> rm = raw(kb - 1);
+        const T wm = w_at(kb - 1);
+        d = der(r0, rm, r1.w, kb);
+        dm = Der9<T>{rm.ux, rm.uy, (T)0, rm.vx, rm.vy, (T)0, rm.wx, rm.wy, rdz * (r0.w - wm)};
+    }
+    Der9<T> dp{};
+    dp.wx = r1.wx;
+    dp.wy = r1.wy;
+    Sij6<T> s0 = sij_of(dm, d, dp, kb, nz);
+    T nk = smag_norm(s0.s11, s0.s12, s0.s13, s0.s22, s0.s23, s0.s33) *
+           a.Cs[base + (long)kb * P] * a.l2;
+    T cs1 = a.Cs[base + (long)k1 * P];
+#pragma unroll
+    for (int q = 0; q < SIJ_L; ++q) {
+        const int k = kb + q;
+        if (k <= min(ke, nz - 1)) {
+            const long o = base + (long)k * P;
+            Raw9<T> r2{};
+            T cs2 = (T)0, w3 = (T)0;
+            if (k + 2 <= min(ke + 1, nz)) {
+                r2 = raw(k + 2);
+                r2.w = w2;
+                cs2 = a.Cs[o + 2 * P];
+                w3 = w_at(min(k + 3, nz));
+            }
+            const Der9<T> d1 = der(r1, r0, w2, k + 1);
+            const Sij6<T> s1 = sij_of(d, d1, d1, k + 1, nz);
+            const T nk1 = smag_norm(s1.s11, s1.s12, s1.s13, s1.s22, s1.s23, s1.s33) * cs1 * a.l2;
+            if (k == 1) {
+                const T c = (T)-2 * (nk + nu);
+                a.txx[o] = c * s0.s11;
+                a.txy[o] = c * s0.s12;
+                a.tyy[o] = c * s0.s22;
+                a.tzz[o] = c * s0.s33;
+            } else if (k == nz - 1) {
+                const T c = (T)0.5 * (nk + nk1) + nu;
+                const T c2 = (T)2 * (nk + nu);
+                a.txx[o] = -c * (s0.s11 + s1.s11);
+                a.txy[o] = -c * (s0.s12 + s1.s12);
+                a.tyy[o] = -c * (s0.s22 + s1.s22);
+                a.tzz[o] = -c * (s0.s33 + s1.s33);
+                a.txz[o] = -c2 * s0.s13;
+                a.tyz[o] = -c2 * s0.s23;
+            } else {
+                const T c = (T)-0.5 * (nk + nk1);
+                const T c2 = (T)-2 * nk;
+                const T c3 = (T)-2 * nu * (T)0.5;
+                const T c4 = (T)-2 * nu;
+                a.txx[o] = (c + c3) * (s0.s11 + s1.s11);
+                a.txy[o] = (c + c3) * (s0.s12 + s1.s12);
+                a.tyy[o] = (c + c3) * (s0.s22 + s1.s22);
+                a.tzz[o] = (c + c3) * (s0.s33 + s1.s33);
+                a.txz[o] = (c2 + c4) * s0.s13;
+                a.tyz[o] = (c2 + c4) * s0.s23;
+            }
+            d = d1;
+            s0 = s1;
+            nk = nk1;
+            r0 = r1;
+            r1 = r2;
+            w2 = w3;
+            cs1 = cs2;
+        }
+    }
+}
+
 // divstress_uv sum (divstress_uv.f90:58-83): k = 1..nz-1, all ld columns;
 // dxy holds ddx(t_x1) + ddy(t_x2) formed in spectral space.
 template <typename T>
