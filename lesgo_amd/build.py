@@ -13,8 +13,9 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "liblesgo_amd.so")
-SOURCES = ["case.hip", "passes_f64.hip", "passes_f32.hip", "tune.hip", "turbines.hip", "capi.hip",
-           "server.hip", "stats.hip", "calibrate.hip", "tridag.hip"]
+SOURCES = ["case.hip", "passes_f64.hip", "passes_f64_cols.hip", "passes_f64_fused.hip",
+           "passes_f32.hip", "passes_f32_cols.hip", "passes_f32_fused.hip", "tune.hip",
+           "turbines.hip", "capi.hip", "server.hip", "stats.hip", "calibrate.hip", "tridag.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

@@ -510,11 +510,12 @@ static void col_common(ColArgs<T>& c, const Dims& d, const T* G1, const T* G2) {
 template <typename T>
 void Case<T>::fwd2d(int njobs, const T* const* src, const T* scales, long src_plane, int src_lev0,
                     long src_ms, cplx<T>* const* dst, long dst_plane, int dst_lev0, long dst_ms,
-                    int nlev, const double* mscale, int band_nzc, int band_ykeep) {
+                    int nlev, const double* mscale, int band_nzc, int band_ykeep,
+                    const int* nl) {
     if (nlev <= 0) return;
     launch_rows_r2c<T>(timer, px.plan, njobs, src, scales, src_plane, d.ld, src_lev0, src_ms, dst,
                        dst_plane, dst_lev0, dst_ms, d.ny, d.NK, nlev, Ma, stream, nullptr,
-                       mscale, CK_N, band_nzc);
+                       mscale, CK_N, band_nzc, nl);
     for (int j0 = 0; j0 < njobs; j0 += MAX_JOBS) {
         const int nj = std::min(MAX_JOBS, njobs - j0);
         ColArgs<T> c{};
@@ -525,6 +526,7 @@ void Case<T>::fwd2d(int njobs, const T* const* src, const T* scales, long src_pl
             c.op[i] = OP_NONE;
             c.nzc[i] = band_nzc;
             c.ykeep[i] = band_ykeep;
+            c.nl[i] = nl ? nl[j0 + i] : 0;
         }
         c.src_plane = c.dst_plane = dst_plane;
         c.lev0_src = c.lev0_dst = dst_lev0;
@@ -539,7 +541,8 @@ void Case<T>::fwd2d(int njobs, const T* const* src, const T* scales, long src_pl
 template <typename T>
 void Case<T>::inv2d(int njobs, const cplx<T>* const* src, const int* ops, long src_plane,
                     int src_lev0, long src_ms, T* const* dst, long dst_plane, int dst_lev0,
-                    long dst_ms, int nlev, cplx<T>* const* tmpspec, const cplx<T>* const* src2) {
+                    long dst_ms, int nlev, cplx<T>* const* tmpspec, const cplx<T>* const* src2,
+                    const int* nl) {
     if (nlev <= 0) return;
     // column-pass output goes to tmpspec[i], planes 0..nlev-1, members packed
     const long tms = (long)nlev * d.splane;
@@ -555,7 +558,7 @@ void Case<T>::inv2d(int njobs, const cplx<T>* const* src, const int* ops, long s
         bool taken[MAX_JOBS] = {};
         T* rdst[MAX_JOBS] = {};
         T* rdst2[MAX_JOBS] = {};
-        int nce[MAX_JOBS] = {};
+        int nce[MAX_JOBS] = {}, rnl[MAX_JOBS] = {};
         for (int i = 0; i < nj; ++i) {
             if (taken[i]) continue;
             c.src[nc] = src[j0 + i];
@@ -563,6 +566,7 @@ void Case<T>::inv2d(int njobs, const cplx<T>* const* src, const int* ops, long s
             c.dst[nc] = tmpspec[nc];
             c.op[nc] = ops[j0 + i];
             rdst[nc] = dst[j0 + i];
+            c.nl[nc] = rnl[nc] = nl ? nl[j0 + i] : 0;
             const bool g1 = ops[j0 + i] == OP_G1 || ops[j0 + i] == OP_G1B;
             nce[nc] = g1 ? g_nzc[0] : ops[j0 + i] == OP_G2 ? g_nzc[1] : 0;
             if (g1 || ops[j0 + i] == OP_G2) {
@@ -594,10 +598,19 @@ void Case<T>::inv2d(int njobs, const cplx<T>* const* src, const int* ops, long s
         c.zero_nyq = 0;
         col_common(c, d, G1, G2);
         launch_cols<T, +1>(timer, c, nc, nlev, Ma, d.ny, stream, nullptr);
+        // the row pass: the jobs of every plane in one launch, then the ones of
+        // a few planes that rode with them (last in the list), over their band
         std::vector<const cplx<T>*> ts(tmpspec, tmpspec + nc);
-        launch_rows_c2r<T>(timer, px.plan, nc, ts.data(), d.splane, 0, tms, rdst, dst_plane,
-                           d.ld, dst_lev0, dst_ms, d.ny, d.NK, nlev, Ma, stream, nullptr, nce,
-                           rdst2, (T)(2.0 * PI_D / d.prm.lx));
+        int nf = nc;
+        while (nf > 0 && rnl[nf - 1]) --nf;
+        for (int f = 0; f < 2; ++f) {
+            const int i0 = f ? nf : 0, n = f ? nc - nf : nf;
+            if (n > 0)
+                launch_rows_c2r<T>(timer, px.plan, n, ts.data() + i0, d.splane, 0, tms, rdst + i0,
+                                   dst_plane, d.ld, dst_lev0, dst_ms, d.ny, d.NK,
+                                   f ? rnl[nf] : nlev, Ma, stream, nullptr, nce + i0, rdst2 + i0,
+                                   (T)(2.0 * PI_D / d.prm.lx));
+        }
     }
 }
 
@@ -768,6 +781,13 @@ void Case<T>::filt_da(int f, int dfdx, int dfdy, cplx<T>* keep) {
 // filt_da (derivatives.f90:166-211) of u, v and w: the three forward
 // transforms in one pass pair, the nine inverses (filtered field, d/dx, d/dy
 // of each) in another; the spectra are kept in sU, sV, sW for convec.
+// forward = false (the spectral-resident step): sU, sV, sW hold the spectra,
+// normalised by 1/(nx ny), and the wall model's test-filtered u, v of level 1
+// (into tmp[0], tmp[1], level 0) ride with the inverses as jobs of one plane:
+// the G_test band of the same spectra (the reference's filtered plane to
+// rounding: G_test is 1/(nx ny) inside a sharp band and zero outside it and on
+// the Nyquist row; the band mask also drops the kx Nyquist column, which the
+// physical u, v do not carry).  A column launch of their own took 4 us.
 template <typename T>
 void Case<T>::filt_da_uvw(bool forward) {
     const T sc = (T)(1.0 / (d.nx * d.ny));
@@ -775,12 +795,14 @@ void Case<T>::filt_da_uvw(bool forward) {
     const T scs[3] = {sc, sc, sc};
     cplx<T>* S[3] = {sU, sV, sW};
     if (forward) fwd2d(3, src, scs, d.plane, 0, d.field, S, d.splane, 0, msp, d.nz + 1);
-    const cplx<T>* is[9] = {sU, sU, sU, sV, sV, sV, sW, sW, sW};
-    const int ops[9] = {OP_NONE, OP_IKX, OP_IKY, OP_NONE, OP_IKX, OP_IKY,
-                        OP_NONE, OP_IKX, OP_IKY};
-    T* dst[9] = {fld[LG_U], fld[LG_DUDX], fld[LG_DUDY], fld[LG_V], fld[LG_DVDX],
-                 fld[LG_DVDY], fld[LG_W], fld[LG_DWDX], fld[LG_DWDY]};
-    inv2d(9, is, ops, d.splane, 0, msp, dst, d.plane, 0, d.field, d.nz + 1, spec);
+    const cplx<T>* is[11] = {sU, sU, sU, sV, sV, sV, sW, sW, sW, sU + d.splane, sV + d.splane};
+    const int ops[11] = {OP_NONE, OP_IKX, OP_IKY, OP_NONE, OP_IKX, OP_IKY,
+                         OP_NONE, OP_IKX, OP_IKY, OP_G1B,  OP_G1B};
+    T* dst[11] = {fld[LG_U],    fld[LG_DUDX], fld[LG_DUDY], fld[LG_V], fld[LG_DVDX], fld[LG_DVDY],
+                  fld[LG_W],    fld[LG_DWDX], fld[LG_DWDY], tmp[0],    tmp[1]};
+    const int nl[11] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 1, 1};
+    inv2d(forward ? 9 : 11, is, ops, d.splane, 0, msp, dst, d.plane, 0, d.field, d.nz + 1, spec,
+          nullptr, nl);
 }
 
 template <typename T>
@@ -896,37 +918,31 @@ void Case<T>::test_filter_plane(const T* in, T* out, int op) {
 // ---------------------------------------------------------------------------
 // wallstress.f90 (lbc_mom = 2, ubc_mom = 0)
 // ---------------------------------------------------------------------------
-// su, sv (the spectral-resident step): the velocity spectra, normalised by
-// 1/(nx ny), whose inverse is the step's u, v; the test filter of the wall
-// level is then their G_test band, with no forward transform (the same
-// values to rounding: G_test is 1/(nx ny) inside a sharp band and zero
-// outside it and on the Nyquist row; the band mask also drops the kx Nyquist
-// column, which the physical u, v do not carry).
 template <typename T>
-void Case<T>::wallstress(const cplx<T>* su, const cplx<T>* sv, bool fill) {
+void Case<T>::wallstress(bool fill) {
     const T one = (T)1;
+    const T* src[2] = {lev(LG_U, 1), lev(LG_V, 1)};
+    const T sc[2] = {one, one};
+    cplx<T>* S0[2] = {spec[4], spec[5]};
+    fwd2d(2, src, sc, d.plane, 0, d.field, S0, d.splane, 0, msp, 1);
     const cplx<T>* s2[2] = {spec[4], spec[5]};
-    int ops[2] = {OP_G1, OP_G1};
-    if (su && sv) {
-        s2[0] = su + d.splane;
-        s2[1] = sv + d.splane;
-        ops[0] = ops[1] = OP_G1B;
-    } else {
-        const T* src[2] = {lev(LG_U, 1), lev(LG_V, 1)};
-        const T sc[2] = {one, one};
-        cplx<T>* S0[2] = {spec[4], spec[5]};
-        fwd2d(2, src, sc, d.plane, 0, d.field, S0, d.splane, 0, msp, 1);
-    }
+    const int ops[2] = {OP_G1, OP_G1};
     T* dst[2] = {tmp[0], tmp[1]};
     cplx<T>* tsp[2] = {spec[6], spec[7]};
     inv2d(2, s2, ops, d.splane, 0, msp, dst, d.plane, 0, d.field, 1, tsp);
+    wall_lbc();
+    if (fill)
+        fill_levels({{LG_TXZ, d.nz, 0.0}, {LG_TYZ, d.nz, 0.0}, {LG_DUDZ, d.nz, 0.0},
+                     {LG_DVDZ, d.nz, 0.0}});
+}
+
+// The wall model from the test-filtered u, v of level 1 in tmp[0], tmp[1].
+template <typename T>
+void Case<T>::wall_lbc() {
     hipLaunchKernelGGL(k_wall_lbc<T>, grid_ij(d.nx, d.ny, 1, Ma), dim3(BLK), 0, stream,
                        (const T*)tmp[0], (const T*)tmp[1], d.field, (const T*)fld[LG_U],
                        (const T*)fld[LG_V], fld[LG_TXZ], fld[LG_TYZ], fld[LG_DUDZ], fld[LG_DVDZ],
                        GEO(1, 1), (const double*)d_denom, d.prm.vonk, d.dz);
-    if (fill)
-        fill_levels({{LG_TXZ, d.nz, 0.0}, {LG_TYZ, d.nz, 0.0}, {LG_DUDZ, d.nz, 0.0},
-                     {LG_DVDZ, d.nz, 0.0}});
 }
 
 // ---------------------------------------------------------------------------
@@ -1266,7 +1282,7 @@ void Case<T>::divstress_uvw() {
 // convec.f90
 // ---------------------------------------------------------------------------
 template <typename T>
-void Case<T>::convec(bool reuse_spectra, bool spectral_out) {
+void Case<T>::convec(bool reuse_spectra, bool spectral_out, const cplx<T>* const* dwall) {
     const T c = (T)(1.0 / (d.nx * d.ny));
     const int nl = d.nz;
     const cplx<T>* ps[6] = {spec[0], spec[1], spec[2], spec[3], spec[4], spec[5]};
@@ -1274,15 +1290,18 @@ void Case<T>::convec(bool reuse_spectra, bool spectral_out) {
         // u, v, w spectra are the ones filt_da just produced (the filtered
         // fields' transforms); the vorticity is formed from them in spectral
         // space, with only the wall-level dvdz/dudz planes transformed (into
-        // planes 0 and 1 of spec[6]).
-        const T* wsrc[2] = {lev(LG_DVDZ, 1), lev(LG_DUDZ, 1)};
-        const T wsc[2] = {c, c};
+        // planes 0 and 1 of spec[6]; or dwall).
         cplx<T>* wd[2] = {spec[6], spec[6] + d.splane};
-        fwd2d(2, wsrc, wsc, d.plane, 0, d.field, wd, d.splane, 0, msp, 1);
+        if (!dwall) {
+            const T* wsrc[2] = {lev(LG_DVDZ, 1), lev(LG_DUDZ, 1)};
+            const T wsc[2] = {c, c};
+            fwd2d(2, wsrc, wsc, d.plane, 0, d.field, wd, d.splane, 0, msp, 1);
+        }
+        const cplx<T>* dw[2] = {dwall ? dwall[0] : wd[0], dwall ? dwall[1] : wd[1]};
         const int n = d.ny * d.NK;
         hipLaunchKernelGGL(k_vort_spec<T>, dim3((n + BLK - 1) / BLK, nl * Ma), dim3(BLK), 0,
                            stream, (const cplx<T>*)sU, (const cplx<T>*)sV, (const cplx<T>*)sW,
-                           (const cplx<T>*)spec[6], (const cplx<T>*)(spec[6] + d.splane), spec[3],
+                           dw[0], dw[1], spec[3],
                            spec[4], spec[5], d.ny, d.NK, d.nz, d.splane,
                            (T)(2.0 * PI_D / d.prm.lx), (T)(2.0 * PI_D / d.prm.ly),
                            (T)(1.0 / d.dz), msp);
@@ -1434,7 +1453,7 @@ void Case<T>::step_body() {
     fill_const_planes();
     filt_da_uvw();
     ddz_uvw();
-    wallstress(nullptr, nullptr, false);
+    wallstress(false);
     sgs_stag(false);
     divstress_uvw();
     convec(true);
@@ -1518,21 +1537,24 @@ void Case<T>::advance_clocks() {
 // Spectral-resident step (spectral.hpp)
 // ---------------------------------------------------------------------------
 // The six stress spectra (levels 1..nz) for divstress_uv + divstress_w,
-// which k_spec_ab2 forms from them; no inverse transform.
+// which k_column forms from them, into spec[6..11]; no inverse transform.
+// The wall level's dvdz, dudz planes, which convec's vorticity takes, ride
+// along as jobs of one plane (level 1 of dwall[0], dwall[1] less a plane: the
+// pass writes level 1 on; launches of their own took 3.6 + 3.3 us at 32^3).
 template <typename T>
-void Case<T>::divstress_spec() {
-    // the stress spectra go to spec[3..8] (convec has finished with them;
-    // its advection spectra stay in spec[0..2]); k_spec_ab2 forms divt
+void Case<T>::divstress_spec(cplx<T>* const* dwall) {
     const T sc = (T)(1.0 / (d.nx * d.ny));
-    const T* src[6] = {fld[LG_TXX], fld[LG_TXY], fld[LG_TYY],
-                       fld[LG_TXZ], fld[LG_TYZ], fld[LG_TZZ]};
-    const T scs[6] = {sc, sc, sc, sc, sc, sc};
-    cplx<T>* S[6] = {spec[3], spec[4], spec[5], spec[6], spec[7], spec[8]};
-    fwd2d(6, src, scs, d.plane, 1, d.field, S, d.splane, 1, msp, d.nz);
+    const T* src[8] = {fld[LG_TXX], fld[LG_TXY], fld[LG_TYY],  fld[LG_TXZ],
+                       fld[LG_TYZ], fld[LG_TZZ], fld[LG_DVDZ], fld[LG_DUDZ]};
+    const T scs[8] = {sc, sc, sc, sc, sc, sc, sc, sc};
+    cplx<T>* S[8] = {spec[6], spec[7],  spec[8],  spec[9],
+                     spec[10], spec[11], dwall[0] - d.splane, dwall[1] - d.splane};
+    const int nl[8] = {0, 0, 0, 0, 0, 0, 1, 1};
+    fwd2d(8, src, scs, d.plane, 1, d.field, S, d.splane, 1, msp, d.nz, nullptr, 0, 0, nl);
 }
 
 // The AB2 update, the pressure solve and the projection on the spectra:
-// advection in spec[0..2], stresses in spec[3..8], u, v, w in sU, sV, sW;
+// advection in spec[0..2], stresses in spec[6..11], u, v, w in sU, sV, sW;
 // p_hat into sP.  One launch (k_column) where the grid has a plan for it, else
 // the separate kernels (k_tridag scales u*, v*, w* by 1/(tadv1 dt) and takes
 // the divtz spectra of levels 1 and nz from sDz).
@@ -1615,10 +1637,12 @@ void Case<T>::step_body_spec(bool cold) {
     filt_da_uvw(false);
     // the stress pass forms d/dz of u, v, w itself; the dynamic model reads them
     if (lag_now) ddz_uvw();
-    wallstress(sU, sV, false);
+    wall_lbc();
     sgs_stag(false, true);
-    convec(true, true);
-    divstress_spec();
+    // the stress spectra in spec[6..11], the wall planes' in spec[0] (levels 1, 2)
+    cplx<T>* dwall[2] = {spec[0] + d.splane, spec[0] + 2 * d.splane};
+    divstress_spec(dwall);
+    convec(true, true, dwall);
     const bool tb = turb && turb->total_nodes > 0 && kf1 >= kf0;
     if (tb) {
         turbines_forcing();
@@ -1627,7 +1651,7 @@ void Case<T>::step_body_spec(bool cold) {
         fwd2d(3, fs, scs, d.plane, kf0, d.field, sF, d.splane, kf0, msp, kf1 - kf0 + 1);
     }
     SpecAb2<T> a{spec[0], spec[1], spec[2],
-                 StressSpec<T>{spec[3], spec[4], spec[5], spec[6], spec[7], spec[8]}, sDz,
+                 StressSpec<T>{spec[6], spec[7], spec[8], spec[9], spec[10], spec[11]}, sDz,
                  (T)(1.0 / d.dz),
                  tb ? sF[0] : nullptr, tb ? sF[1] : nullptr, tb ? sF[2] : nullptr,
                  sR[0], sR[1], sR[2], sRf[0], sRf[1], sRf[2], sPf, sU, sV, sW, d_mpf,

@@ -215,14 +215,16 @@ struct Case {
     T* mem(int id, int m) { return fld[id] + (long)m * d.field; }
 
     // 2-D transform helpers over planes [lev0, lev0+nlev) of every member
-    // band (nzc, ykeep; 0: none): the spectra are only read inside the test
+    // nl: planes of each job (null or 0: nlev); band (nzc, ykeep; 0: none): the spectra are only read inside the test
     // filters' band, so only that part is computed and written
     void fwd2d(int njobs, const T* const* src, const T* scales, long src_plane, int src_lev0,
                long src_ms, cplx<T>* const* dst, long dst_plane, int dst_lev0, long dst_ms,
-               int nlev, const double* mscale = nullptr, int band_nzc = 0, int band_ykeep = 0);
+               int nlev, const double* mscale = nullptr, int band_nzc = 0, int band_ykeep = 0,
+               const int* nl = nullptr);
     void inv2d(int njobs, const cplx<T>* const* src, const int* ops, long src_plane, int src_lev0,
                long src_ms, T* const* dst, long dst_plane, int dst_lev0, long dst_ms, int nlev,
-               cplx<T>* const* tmpspec, const cplx<T>* const* src2 = nullptr);
+               cplx<T>* const* tmpspec, const cplx<T>* const* src2 = nullptr,
+               const int* nl = nullptr);
     void pad_inv_big(int njobs, const cplx<T>* const* src, int lev0, int nlev);
     void fwd_big_unpad(int njobs, const T* const* src, cplx<T>* const* dst, int lev0, int nlev);
     void cols_unpad(int njobs, cplx<T>* const* dst, int lev0, int nlev);
@@ -237,8 +239,9 @@ struct Case {
     void ddz_uvw();        // ddz_uv(u), ddz_uv(v), ddz_w(w): one pass, the same values
     void test_filter_plane(const T* in, T* out, int op);
     void fill_const_planes();
-    // fill: set the lid's (ghost) planes too (a step has set them already)
-    void wallstress(const cplx<T>* su = nullptr, const cplx<T>* sv = nullptr, bool fill = true);
+    // fill: set the ghost and lid planes too (a step has set them already)
+    void wallstress(bool fill = true);
+    void wall_lbc();
     void calc_sij();
     // from_uvw: without a dynamic-model update, form d/dz of u, v, w in the pass
     void sgs_stag(bool fill = true, bool from_uvw = false);
@@ -250,7 +253,9 @@ struct Case {
     // divstress routines with one forward and one inverse pass
     void filt_da_uvw(bool forward = true);
     void divstress_uvw();
-    void convec(bool reuse_spectra = false, bool spectral_out = false);
+    // dwall: spectra of the wall level's dvdz, dudz planes (null: made here)
+    void convec(bool reuse_spectra = false, bool spectral_out = false,
+                const cplx<T>* const* dwall = nullptr);
     void press_stag_array();
     void project();
     void rhs_ab2();
@@ -269,7 +274,7 @@ struct Case {
     void copy_spec_member(int src, int dst);
     void run_body(bool cold);
     void after_body();
-    void divstress_spec();
+    void divstress_spec(cplx<T>* const* dwall);
     void column_spec(const SpecAb2<T>& a);
     void materialize(unsigned groups);
     void touch(bool modify);

@@ -231,6 +231,8 @@ struct RowR2CArgs {
     int mscale_stride;
     int nwr;               // columns of dst written (0: ncols; a band-limited consumer
                            // reads no more; the four-step and generic kernels honour it)
+    int nl[MAX_JOBS];      // planes of the job (0: nlev): a job of few planes rides with
+                           // others in one launch, its blocks past them end at once
 };
 
 // The fields the convective products are formed from (prod_rows.hpp): u, v,
@@ -250,6 +252,7 @@ __global__ void __launch_bounds__(256) k_rows_r2c(RowR2CArgs<T> a) {
     const int job = blockIdx.z;
     const int mem = blockIdx.y / a.nlev;
     const int plane = blockIdx.y - mem * a.nlev;
+    if (a.nl[job] && plane >= a.nl[job]) return;
     const int npairs = a.nrows / 2;
     const int pair0 = blockIdx.x * a.S;
     const int S = min(a.S, npairs - pair0);
@@ -454,6 +457,7 @@ struct ColArgs {
     // inverse MAP_ID jobs: the input's ky = ny/2 row is taken as zero (as
     // filt_da's is) when set
     int nyq0[MAX_JOBS];
+    int nl[MAX_JOBS];  // planes of the job (0: nlev), as RowR2CArgs
 };
 
 // Row jb of a small-grid spectrum inside the band |m| < ykeep (0: all rows).
@@ -511,6 +515,7 @@ __global__ void __launch_bounds__(256) k_cols(ColArgs<T> a) {
     const int ykeep = a.ykeep[job];
     const int mem = blockIdx.z / a.nlev;
     const int plane = blockIdx.z - mem * a.nlev;
+    if (a.nl[job] && plane >= a.nl[job]) return;
     const cplx<T>* src = a.src[job] + mem * a.src_mstride + (long)(a.lev0_src + plane) * a.src_plane;
     cplx<T>* dst = a.dst[job] + mem * a.dst_mstride + (long)(a.lev0_dst + plane) * a.dst_plane;
     const int op = a.op[job];

@@ -304,16 +304,19 @@ void launch_rows_r2c(KernelTimer& tm, const FftPlan& pl, int njobs, const T* con
                      const T* scales, long src_plane, int src_ld, int src_lev0, long src_ms,
                      cplx<T>* const* dst, long dst_plane, int dst_lev0, long dst_ms, int nrows,
                      int ncols, int nlev, int M, hipStream_t s, const PassChoice* force,
-                     const double* mscale, int mscale_stride, int nwr) {
+                     const double* mscale, int mscale_stride, int nwr, const int* nl) {
     const PassChoice ch = force ? *force : choice_for<T>(PK_R2C, pl.N, nrows);
     for (int j0 = 0; j0 < njobs; j0 += MAX_JOBS) {
         const int nj = std::min(MAX_JOBS, njobs - j0);
         RowR2CArgs<T> a{};
         a.plan = pl;
+        double planes = 0.0;   // summed over the jobs
         for (int i = 0; i < nj; ++i) {
             a.src[i] = src[j0 + i];
             a.dst[i] = dst[j0 + i];
             a.scale[i] = scales ? scales[j0 + i] : (T)1;
+            a.nl[i] = nl ? nl[j0 + i] : 0;
+            planes += a.nl[i] ? a.nl[i] : nlev;
         }
         a.src_plane = src_plane;
         a.dst_plane = dst_plane;
@@ -332,7 +335,7 @@ void launch_rows_r2c(KernelTimer& tm, const FftPlan& pl, int njobs, const T* con
         a.stride = seq_stride(ch, pl.N);
         const size_t lds = row_lds_bytes<T>(ch, pl.N, src_ld, ncols);
         dim3 grid((nrows / 2 + a.S - 1) / a.S, nlev * M, nj);
-        const double bytes = (double)nj * nlev * M * nrows *
+        const double bytes = planes * M * nrows *
                              ((double)pl.N * sizeof(T) + (double)(a.nwr ? a.nwr : ncols) * sizeof(cplx<T>));
         tm.run(s, 3 * ncols == pl.N ? KK_ROWS_R2C_PAD : KK_ROWS_R2C, bytes, [&] {
             if (ch.n1 && ch.v == 1 && v3_r2c<T>(ch.n1, ch.n2, grid, lds, s, a)) return;
@@ -414,7 +417,7 @@ void launch_cols(KernelTimer& tm, ColArgs<T>& c, int nj, int nlev, int M, int ny
     // band-limited jobs: columns < nzc, and (MAP_ID) rows |ky| < ykeep read by
     // an inverse pass or written by a forward one
     int cmax = 0;
-    double cols_rw = 0.0;      // sum over jobs of columns x rows moved
+    double cols_rw = 0.0;      // sum over jobs of planes x columns x rows moved
     for (int i = 0; i < nj; ++i) {
         const int nzc = (c.nzc[i] > 0 && c.nzc[i] < c.ncols) ? c.nzc[i] : c.ncols;
         c.nzc[i] = nzc < c.ncols ? nzc : 0;
@@ -423,10 +426,10 @@ void launch_cols(KernelTimer& tm, ColArgs<T>& c, int nj, int nlev, int M, int ny
         const double rin = (DIR > 0 && band) ? band : ny_in;
         // MAP_UNPAD writes the small grid's ny rows, not the N it transforms
         const double rout = c.map == MAP_UNPAD ? c.ny : ((DIR < 0 && band) ? band : N);
-        cols_rw += (double)nzc * (rin + rout);
+        cols_rw += (double)(c.nl[i] ? c.nl[i] : nlev) * nzc * (rin + rout);
     }
     dim3 grid(nj, (cmax + c.TC - 1) / c.TC, nlev * M);
-    const double bytes = (double)nlev * M * sizeof(cplx<T>) * cols_rw;
+    const double bytes = (double)M * sizeof(cplx<T>) * cols_rw;
     const int kk = c.map == MAP_PAD ? KK_COLS_PAD
                    : (c.map == MAP_UNPAD ? KK_COLS_UNPAD : (DIR < 0 ? KK_COLS_FWD : KK_COLS_INV));
     tm.run(s, kk, bytes, [&] {
