@@ -24,12 +24,26 @@ constexpr int TRI_STATUS_INTS = 64;
 // system (tridag_array.f90:190-200); rows 2..nz+1 skip jy = ny/2+1 and
 // (jx, jy) = (1, 1) as the reference does (207-209), leaving those entries
 // of u as they were.  gam holds the forward-sweep ratios (lh, ny, nz+1).
-__global__ void __launch_bounds__(256) k_tridag_array(const double* __restrict__ a,
-                                                      const double* __restrict__ b,
-                                                      const double* __restrict__ c,
-                                                      const double2* __restrict__ r,
-                                                      double2* __restrict__ u, double* gam,
-                                                      int lh, int ny, int n, int* status) {
+//
+// Bound by latency: 128 x 256 systems are half a wave a SIMD, so a sweep that
+// waits for each row's loads pays the memory's latency at every row.  A block
+// of TRA_BLK rows is therefore solved in registers while the next block's
+// loads, issued together and unconditionally, are in flight; its results are
+// stored after the block (a store under a condition between the loads would
+// make the compiler wait for all of them: a ring of rows loaded one by one
+// stayed at 258 us).  One wave a block puts the systems on all CUs.  The
+// arithmetic and its order are the plain recurrence's.  The whole device call,
+// row at a time and 256 threads a block -> this: 129 x 256 x 193 380 -> 190 us,
+// 65 x 128 x 97 159 -> 91, 33 x 64 x 65 73 -> 50, 9 x 16 x 11 33 -> 33 (of which
+// about 45 are the allocation, the status read and the launch).  Blocks of 4
+// rows 195, of 6 191, of 12 191 us at the first.
+constexpr int TRA_BLK = 8;
+constexpr int TRA_THREADS = 64;
+
+__global__ void __launch_bounds__(TRA_THREADS) k_tridag_array(
+    const double* __restrict__ a, const double* __restrict__ b, const double* __restrict__ c,
+    const double2* __restrict__ r, double2* u, double* gam, int lh, int ny, int n, int* status) {
+    constexpr int B = TRA_BLK;
     const int gid = blockIdx.x * blockDim.x + threadIdx.x;
     const int nsys = (lh - 1) * ny;
     if (gid >= nsys) return;
@@ -54,26 +68,76 @@ __global__ void __launch_bounds__(256) k_tridag_array(const double* __restrict__
     u[o] = up;
     if (jy == ny / 2 || (jx == 0 && jy == 0)) return;
     double bet = b0;
-    for (int j = 1; j < n; ++j) {
-        const long oj = (long)j * plane + o;
-        const double gm = c[oj - plane] / bet;
-        gam[oj] = gm;
-        const double aj = a[oj];
-        bet = b[oj] - aj * gm;
-        if (bet == 0.0) {
-            fail(j + 1);
+    // rows j0 .. j0 + B - 1 of the coefficients (indices clamped to the last row)
+    struct Rows {
+        double a[B], b[B], c[B];
+        double2 r[B];
+    } cur, nxt;
+    auto load = [&](int j0, Rows& q) {
+#pragma unroll
+        for (int i = 0; i < B; ++i) {
+            const long oj = (long)min(j0 + i, n - 1) * plane + o;
+            q.a[i] = a[oj];
+            q.b[i] = b[oj];
+            q.c[i] = c[oj - plane];
+            q.r[i] = r[oj];
+        }
+    };
+    load(1, cur);
+    for (int j0 = 1; j0 < n; j0 += B) {
+        load(j0 + B, nxt);
+        double gm[B];
+        double2 ub[B];
+        int end = n;                  // rows from the first zero pivot on are not written
+#pragma unroll
+        for (int i = 0; i < B; ++i) {
+            gm[i] = cur.c[i] / bet;
+            const double aj = cur.a[i];
+            const double bj = cur.b[i] - aj * gm[i];
+            if (bj == 0.0 && j0 + i < end) end = j0 + i;
+            const double2 rj = cur.r[i];
+            ub[i] = make_double2((rj.x - aj * up.x) / bj, (rj.y - aj * up.y) / bj);
+            if (j0 + i < n) {
+                bet = bj;
+                up = ub[i];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < B; ++i)
+            if (j0 + i < end) {
+                gam[(long)(j0 + i) * plane + o] = gm[i];
+                u[(long)(j0 + i) * plane + o] = ub[i];
+            }
+        if (end < n) {
+            fail(end + 1);
             return;
         }
-        const double2 rj = r[oj];
-        up = make_double2((rj.x - aj * up.x) / bet, (rj.y - aj * up.y) / bet);
-        u[oj] = up;
+        cur = nxt;
     }
-    for (int j = n - 2; j >= 0; --j) {
-        const long oj = (long)j * plane + o;
-        const double gm = gam[oj + plane];
-        const double2 uj = u[oj];
-        up = make_double2(uj.x - gm * up.x, uj.y - gm * up.y);
-        u[oj] = up;
+    // back substitution, rows n - 2 .. 0, loaded ahead alike
+    struct Back {
+        double g[B];
+        double2 u[B];
+    } bc, bn;
+    auto loadb = [&](int j0, Back& q) {
+#pragma unroll
+        for (int i = 0; i < B; ++i) {
+            const long oj = (long)max(j0 - i, 0) * plane + o;
+            q.g[i] = gam[oj + plane];
+            q.u[i] = u[oj];
+        }
+    };
+    loadb(n - 2, bc);
+    for (int j0 = n - 2; j0 >= 0; j0 -= B) {
+        loadb(j0 - B, bn);
+#pragma unroll
+        for (int i = 0; i < B; ++i) {
+            if (j0 - i >= 0) {
+                up = make_double2(bc.u[i].x - bc.g[i] * up.x, bc.u[i].y - bc.g[i] * up.y);
+                u[(long)(j0 - i) * plane + o] = up;
+            }
+        }
+        bc = bn;
     }
 }
 
@@ -91,7 +155,8 @@ int tridag_array_run(int lh, int ny, int n, const double* a, const double* b, co
     hipLaunchKernelGGL(k_clear_ints, dim3(1), dim3(TRI_STATUS_INTS), 0, stream, status,
                        TRI_STATUS_INTS);
     const int nsys = (lh - 1) * ny;
-    hipLaunchKernelGGL(k_tridag_array, dim3((nsys + 255) / 256), dim3(256), 0, stream, a, b, c,
+    hipLaunchKernelGGL(k_tridag_array, dim3((nsys + TRA_THREADS - 1) / TRA_THREADS),
+                       dim3(TRA_THREADS), 0, stream, a, b, c,
                        reinterpret_cast<const double2*>(r), reinterpret_cast<double2*>(u), gam,
                        lh, ny, n, status);
     LG_HIP(hipGetLastError());

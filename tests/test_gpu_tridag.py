@@ -109,3 +109,42 @@ def test_tridag_array_zero_pivot_is_reported(row):
     assert rc == 6                       # LG_ERR_PIVOT
     msg = _lib.lib().lg_last_error().decode()
     assert f"{jx}, {jy}, {row}" in msg, msg
+
+
+# The sweeps work in blocks of 8 rows: the first and last row of a block, and
+# counts of rows just below, at and above whole blocks.
+@pytest.mark.parametrize("n", [3, 8, 9, 10, 16, 17, 18, 25])
+def test_tridag_array_block_edges(n):
+    lh, ny = 9, 4
+    a, b, c, r = systems(lh, ny, n, "random", seed=n)
+    u = np.full_like(r, SENTINEL)
+    assert host_call(lh, ny, n, a, b, c, r, u) == 0
+    ref = oracle_solve(lh, ny, n, a, b, c, r)
+    m = written_mask(lh, ny, n)
+    assert np.linalg.norm(u[m] - ref[m]) <= 1e-13 * np.linalg.norm(ref[m])
+    assert (u[~m] == SENTINEL).all()
+
+
+@pytest.mark.parametrize("row", [8, 9, 10, 18])
+def test_tridag_array_zero_pivot_in_a_later_block(row):
+    """A pivot that vanishes at the given row: reported with it, rows from it
+    on left as they were."""
+    from lesgo_amd import _lib
+    lh, ny, n = 17, 4, 18
+    a, b, c, r = systems(lh, ny, n, "random", seed=row)
+    jx, jy = 5, 2
+    i = (jy - 1, jx - 1)
+    # a = 0 above the row keeps its bet at b = 2, so bet(row) = 2 - 4 c / 2 = 0
+    a[row - 2][i], b[row - 2][i], c[row - 2][i] = 0.0, 2.0, 1.0
+    a[row - 1][i], b[row - 1][i] = 4.0, 2.0
+    u = np.full_like(r, SENTINEL)
+    x = [np.ascontiguousarray(v) for v in (a, b, c, r)]
+    from hip_util import DeviceArray
+    dev = [DeviceArray(v) for v in x]
+    du = DeviceArray(shape=r.shape, fill=SENTINEL)
+    rc = _lib.lib().lg_tridag_array_device(lh, ny, n, *[v.ptr for v in dev], du.ptr, None)
+    assert rc == 6                       # LG_ERR_PIVOT
+    msg = _lib.lib().lg_last_error().decode()
+    assert f"{jx}, {jy}, {row}" in msg, msg
+    got = du.get()[:, jy - 1, 2 * (jx - 1)]
+    assert (got[row - 1:] == SENTINEL).all() and (got[:row - 1] != SENTINEL).all()
