@@ -174,18 +174,7 @@ int lg_download_member(lg_case* h, int m, int field, double* host) {
         check_field(field);
         check_member(c, m);
         REQUIRE(host, "null host pointer");
-        using T = typename std::remove_reference<decltype(*c.fld[0])>::type;
-        if constexpr (std::is_same<T, double>::value) {
-            LG_HIP(hipMemcpyAsync(host, c.mem(field, m), c.d.field * sizeof(double),
-                                  hipMemcpyDeviceToHost, c.stream));
-            LG_HIP(hipStreamSynchronize(c.stream));
-        } else {
-            std::vector<T> tmp((size_t)c.d.field);
-            LG_HIP(hipMemcpyAsync(tmp.data(), c.mem(field, m), c.d.field * sizeof(T),
-                                  hipMemcpyDeviceToHost, c.stream));
-            LG_HIP(hipStreamSynchronize(c.stream));
-            for (long i = 0; i < c.d.field; ++i) host[i] = (double)tmp[i];
-        }
+        c.hcopy.read(c.mem(field, m), host, c.d.field, c.stream);
     });
 }
 

@@ -213,6 +213,7 @@ Case<T>::Case(const lg_params& p, int members) : d(p), M(members), Ma(members) {
     for (int i = 0; i < (prod_fused ? 6 : NBIG); ++i) big[i] = dalloc<T>(M * mbp);
     for (int i = 0; i < 6; ++i) bigspec[i] = dalloc<cplx<T>>(M * mbsp);
     for (int i = 0; i < NTMP; ++i) tmp[i] = dalloc<T>(M * d.field);
+    hcopy.prepare(d.field, sizeof(T));
     gam = dalloc<double>(msp);
     {
         // the elimination coefficients of the pressure systems (grid only)

@@ -8,6 +8,7 @@
 #include "../../include/lesgo_amd.h"
 #include "common.hpp"
 #include "fft.hpp"
+#include "hostcopy.hpp"
 #include "passes.hpp"
 #include "timer.hpp"
 
@@ -90,6 +91,7 @@ struct Case {
     long mbp = 0;                    // (nz+1) * bplane
     long mbsp = 0;                   // (nz+1) * bsplane
     hipStream_t stream = nullptr;
+    HostCopy hcopy;                  // staging of fields read back
     int jt = 0, jt_total = 0;
     bool swapped = false;            // RHS / RHS_f storage exchanged (odd steps)
     std::vector<double> zo, mpf;     // per member z0 and mean_p_force (x, y)

@@ -168,12 +168,9 @@ struct Server {
         p.with([&](auto& c) {
             if (job.keep) {
                 c.touch(false);
-                using T = typename std::remove_reference<decltype(*c.fld[0])>::type;
-                std::vector<T> tmp((size_t)c.d.field);
                 for (int id : {LG_U, LG_V, LG_W, LG_P}) {
-                    LG_HIP(hipMemcpy(tmp.data(), c.mem(id, slot), c.d.field * sizeof(T),
-                                     hipMemcpyDeviceToHost));
-                    job.kept.emplace_back(tmp.begin(), tmp.end());
+                    job.kept.emplace_back((size_t)c.d.field);
+                    c.hcopy.read(c.mem(id, slot), job.kept.back().data(), c.d.field, c.stream);
                 }
             }
             const int last = c.Ma - 1;
