@@ -231,8 +231,11 @@ struct RowR2CArgs {
     int mscale_stride;
     int nwr;               // columns of dst written (0: ncols; a band-limited consumer
                            // reads no more; the four-step and generic kernels honour it)
-    int nl[MAX_JOBS];      // planes of the job (0: nlev): a job of few planes rides with
-                           // others in one launch, its blocks past them end at once
+    // a job of few planes rides with others in one launch (ride set): nl[job] is
+    // its number of planes (0: nlev), its blocks past them end at once.  Without
+    // riders no block waits for the indexed nl before its other loads.
+    int ride;
+    int nl[MAX_JOBS];
 };
 
 // The fields the convective products are formed from (prod_rows.hpp): u, v,
@@ -252,7 +255,7 @@ __global__ void __launch_bounds__(256) k_rows_r2c(RowR2CArgs<T> a) {
     const int job = blockIdx.z;
     const int mem = blockIdx.y / a.nlev;
     const int plane = blockIdx.y - mem * a.nlev;
-    if (a.nl[job] && plane >= a.nl[job]) return;
+    if (a.ride && a.nl[job] && plane >= a.nl[job]) return;
     const int npairs = a.nrows / 2;
     const int pair0 = blockIdx.x * a.S;
     const int S = min(a.S, npairs - pair0);
@@ -457,6 +460,7 @@ struct ColArgs {
     // inverse MAP_ID jobs: the input's ky = ny/2 row is taken as zero (as
     // filt_da's is) when set
     int nyq0[MAX_JOBS];
+    int ride;
     int nl[MAX_JOBS];  // planes of the job (0: nlev), as RowR2CArgs
 };
 
@@ -515,7 +519,7 @@ __global__ void __launch_bounds__(256) k_cols(ColArgs<T> a) {
     const int ykeep = a.ykeep[job];
     const int mem = blockIdx.z / a.nlev;
     const int plane = blockIdx.z - mem * a.nlev;
-    if (a.nl[job] && plane >= a.nl[job]) return;
+    if (a.ride && a.nl[job] && plane >= a.nl[job]) return;
     const cplx<T>* src = a.src[job] + mem * a.src_mstride + (long)(a.lev0_src + plane) * a.src_plane;
     cplx<T>* dst = a.dst[job] + mem * a.dst_mstride + (long)(a.lev0_dst + plane) * a.dst_plane;
     const int op = a.op[job];

@@ -316,6 +316,7 @@ void launch_rows_r2c(KernelTimer& tm, const FftPlan& pl, int njobs, const T* con
             a.dst[i] = dst[j0 + i];
             a.scale[i] = scales ? scales[j0 + i] : (T)1;
             a.nl[i] = nl ? nl[j0 + i] : 0;
+            a.ride |= a.nl[i];
             planes += a.nl[i] ? a.nl[i] : nlev;
         }
         a.src_plane = src_plane;
@@ -417,11 +418,13 @@ void launch_cols(KernelTimer& tm, ColArgs<T>& c, int nj, int nlev, int M, int ny
     // band-limited jobs: columns < nzc, and (MAP_ID) rows |ky| < ykeep read by
     // an inverse pass or written by a forward one
     int cmax = 0;
+    c.ride = 0;
     double cols_rw = 0.0;      // sum over jobs of planes x columns x rows moved
     for (int i = 0; i < nj; ++i) {
         const int nzc = (c.nzc[i] > 0 && c.nzc[i] < c.ncols) ? c.nzc[i] : c.ncols;
         c.nzc[i] = nzc < c.ncols ? nzc : 0;
         cmax = std::max(cmax, nzc);
+        c.ride |= c.nl[i];
         const int band = c.ykeep[i] > 0 ? std::min(2 * c.ykeep[i] - 1, ny_in) : 0;
         const double rin = (DIR > 0 && band) ? band : ny_in;
         // MAP_UNPAD writes the small grid's ny rows, not the N it transforms
