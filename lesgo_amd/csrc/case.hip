@@ -451,7 +451,8 @@ template <typename T>
 void Case<T>::clock_begin() {
     if (!cfl_mode) return;
     const long n = (long)(d.nz - 1) * d.ny * d.nx;
-    const int nb = (int)std::max(1L, std::min(1024L, n / (BLK * 32L)));
+    // four points a thread: with 32, 96 x 48 x 64 gave 36 blocks for 256 CUs
+    const int nb = (int)std::max(1L, std::min(1024L, n / (BLK * 4L)));
     hipLaunchKernelGGL(k_cfl_max<T>, dim3(nb, Ma), dim3(BLK), 0, stream, (const T*)fld[LG_U],
                        (const T*)fld[LG_V], (const T*)fld[LG_W], d.nx, d.ny, d.ld, d.plane,
                        d.field, d.nz, d_cmax);
@@ -1267,16 +1268,10 @@ void Case<T>::divstress_uvw() {
     T* dst[3] = {tmp[0], tmp[2], tmp[4]};
     cplx<T>* tsp[3] = {spec[5], spec[6], spec[7]};
     inv2d(3, is, ops, d.splane, 1, msp, dst, d.plane, 1, d.field, d.nz, tsp, is2);
-    const int nl = d.nz - 1;
-    const T rdz = (T)(1.0 / d.dz);
-    hipLaunchKernelGGL(k_divt_uv<T>, grid_ij(d.ld, d.ny, nl, Ma), dim3(BLK), 0, stream,
-                       (const T*)tmp[0], (const T*)fld[LG_TXZ], fld[LG_DIVTX], GEO(1, nl), rdz);
-    hipLaunchKernelGGL(k_divt_uv<T>, grid_ij(d.ld, d.ny, nl, Ma), dim3(BLK), 0, stream,
-                       (const T*)tmp[2], (const T*)fld[LG_TYZ], fld[LG_DIVTY], GEO(1, nl), rdz);
-    hipLaunchKernelGGL(k_divt_w<T>, grid_ij(d.ld, d.ny, d.nz, Ma), dim3(BLK), 0, stream,
-                       (const T*)tmp[4], (const T*)fld[LG_TZZ], fld[LG_DIVTZ], GEO(1, d.nz), rdz);
-    fill_levels({{LG_DIVTX, 0, BOGUS}, {LG_DIVTX, d.nz, BOGUS}, {LG_DIVTY, 0, BOGUS},
-                 {LG_DIVTY, d.nz, BOGUS}, {LG_DIVTZ, 0, BOGUS}});
+    const DivtArgs<T> a{tmp[0],      tmp[2],      tmp[4],       fld[LG_TXZ],  fld[LG_TYZ],
+                        fld[LG_TZZ], fld[LG_DIVTX], fld[LG_DIVTY], fld[LG_DIVTZ]};
+    hipLaunchKernelGGL(k_divt_uvw<T>, grid_ij(d.ld, d.ny, d.nz + 1, Ma), dim3(BLK), 0, stream, a,
+                       GEO(0, d.nz + 1), (T)(1.0 / d.dz), (T)BOGUS);
 }
 
 // ---------------------------------------------------------------------------
@@ -1352,7 +1347,7 @@ void Case<T>::convec(bool reuse_spectra, bool spectral_out, const cplx<T>* const
 // press_stag_array.f90 + tridag_array.f90
 // ---------------------------------------------------------------------------
 template <typename T>
-void Case<T>::press_stag_array() {
+void Case<T>::press_stag_array(bool dpdz) {
     const double cst = 1.0 / (d.nx * d.ny);
     const T c2 = (T)(cst / d.tadv1 / d.prm.dt);
     {
@@ -1401,6 +1396,7 @@ void Case<T>::press_stag_array() {
         cplx<T>* tsp[2] = {spec[5], spec[6]};
         inv2d(2, is, ops, d.splane, 1, msp, dst, d.plane, 1, d.field, d.nz - 1, tsp);
     }
+    if (!dpdz) return;
     hipLaunchKernelGGL(k_dpdz<T>, grid_ij(d.nx, d.ny, d.nz, Ma), dim3(BLK), 0, stream,
                        (const T*)fld[LG_P], fld[LG_DPDZ], GEO(1, d.nz), (T)d.dz);
     fill_levels({{LG_DPDX, d.nz, BOGUS}, {LG_DPDY, d.nz, BOGUS}});
@@ -1427,7 +1423,7 @@ void Case<T>::project() {
 // main.f90 time loop body
 // ---------------------------------------------------------------------------
 template <typename T>
-void Case<T>::rhs_ab2() {
+void Case<T>::rhs_ab2(bool fill) {
     const bool tb = (bool)turb;
     Ab2Args<T> a{fld[LG_U], fld[LG_V], fld[LG_W], fld[LG_RHSX], fld[LG_RHSY], fld[LG_RHSZ],
                  fld[LG_RHSX_F], fld[LG_RHSY_F], fld[LG_RHSZ_F], fld[LG_DIVTX], fld[LG_DIVTY],
@@ -1436,6 +1432,7 @@ void Case<T>::rhs_ab2() {
                  (const int*)d_flags, d.prm.use_mean_p_force, clk()};
     hipLaunchKernelGGL(k_rhs_ab2<T>, grid_ij(d.ld, d.ny, d.nz, Ma), dim3(BLK), 0, stream, a,
                        GEO(1, d.nz));
+    if (!fill) return;
     fill_levels({{LG_U, 0, BOGUS}, {LG_V, 0, BOGUS}, {LG_W, 0, BOGUS}, {LG_U, d.nz, BOGUS},
                  {LG_V, d.nz, BOGUS}});
 }
@@ -1445,6 +1442,17 @@ void Case<T>::rhs_gradp() {
     hipLaunchKernelGGL(k_rhs_gradp<T>, grid_ij(d.ld, d.ny, d.nz, Ma), dim3(BLK), 0, stream,
                        fld[LG_RHSX], fld[LG_RHSY], fld[LG_RHSZ], (const T*)fld[LG_DPDX],
                        (const T*)fld[LG_DPDY], (const T*)fld[LG_DPDZ], GEO(1, d.nz));
+}
+
+// dpdz, RHS - grad p, project and the planes that rhs_ab2 and press_stag_array
+// leave to it, in one launch (convec sets its own: an Euler step copies them).
+template <typename T>
+void Case<T>::press_tail() {
+    const TailArgs<T> a{fld[LG_U],    fld[LG_V],    fld[LG_W],       fld[LG_RHSX], fld[LG_RHSY],
+                        fld[LG_RHSZ], fld[LG_DPDX], fld[LG_DPDY],    fld[LG_DPDZ], fld[LG_P],
+                        (T)d.prm.dt,  (T)d.tadv1,   (T)d.dz,         (T)BOGUS,     clk()};
+    hipLaunchKernelGGL(k_press_tail<T>, grid_ij(d.ld, d.ny, d.nz + 1, Ma), dim3(BLK), 0, stream,
+                       a, GEO(0, d.nz + 1));
 }
 
 // The loop body after the counters advance and RHS_f = RHS (main.f90:155-326).
@@ -1459,10 +1467,9 @@ void Case<T>::step_body() {
     divstress_uvw();
     convec(true);
     if (turb) turbines_forcing();
-    rhs_ab2();
-    press_stag_array();
-    rhs_gradp();
-    project();
+    rhs_ab2(false);
+    press_stag_array(false);
+    press_tail();
 }
 
 

@@ -258,9 +258,10 @@ struct Case {
     // dwall: spectra of the wall level's dvdz, dudz planes (null: made here)
     void convec(bool reuse_spectra = false, bool spectral_out = false,
                 const cplx<T>* const* dwall = nullptr);
-    void press_stag_array();
+    void press_stag_array(bool dpdz = true);
     void project();
-    void rhs_ab2();
+    void press_tail();               // dpdz, rhs_gradp, project and their planes in one launch
+    void rhs_ab2(bool fill = true);
     void rhs_gradp();
     bool refresh_flags(bool force_lag = false);
     const double* clk() const { return cfl_mode ? d_clock : nullptr; }

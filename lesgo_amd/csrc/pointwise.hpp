@@ -658,6 +658,53 @@ __global__ void k_divt_w(const T* dxy, const T* tzz, T* out, Geo g, T rdz) {
     }
 }
 
+// The z terms and the constant planes of all three divergences in one launch
+// over k = 0..nz and all ld columns: the two sums above and, at the planes they
+// leave out, what divstress_uv and divstress_w leave there.  Bound by the
+// launch on small grids: 96 x 48 x 64 mixed, three sums and a fill of 18.7 us.
+template <typename T>
+struct DivtArgs {
+    const T *dx, *dy, *dw;         // spectral-space sums (ddx + ddy)
+    const T *txz, *tyz, *tzz;
+    T *ox, *oy, *oz;
+};
+
+template <typename T>
+__global__ void k_divt_uvw(DivtArgs<T> a, Geo g, T rdz, T bogus) {
+    int m, k, j, i;
+    long mb;
+    if (!pt_of(g, g.ld, m, k, j, i, mb)) return;
+    const long o = mb + (long)k * g.plane + (long)j * g.ld + i;
+    if (k == 0) {
+        a.ox[o] = bogus;
+        a.oy[o] = bogus;
+        a.oz[o] = bogus;
+        return;
+    }
+    if (k == g.nz) {
+        a.ox[o] = bogus;
+        a.oy[o] = bogus;
+        if (i < g.nx) a.oz[o] = a.dw[o];
+        return;
+    }
+    if (i >= g.nx) {
+        a.ox[o] = (T)0;
+        a.oy[o] = (T)0;
+        a.oz[o] = (T)0;
+        return;
+    }
+    const T zx = rdz * (a.txz[o + g.plane] - a.txz[o]);
+    a.ox[o] = a.dx[o] + zx;
+    const T zy = rdz * (a.tyz[o + g.plane] - a.tyz[o]);
+    a.oy[o] = a.dy[o] + zy;
+    if (k == 1) {
+        a.oz[o] = a.dw[o];
+    } else {
+        const T zz = rdz * (a.tzz[o] - a.tzz[o - g.plane]);
+        a.oz[o] = a.dw[o] + zz;
+    }
+}
+
 // convec vorticity (convec.f90:97-168), scaled by 1/(nx ny), k = 1..nz.
 template <typename T>
 struct VortArgs {
@@ -957,6 +1004,67 @@ __global__ void k_project(T* u, T* v, T* w, const T* px, const T* py, const T* p
     u[o] = u[o] + dt * (-(t1 * px[o]));
     v[o] = v[o] + dt * (-(t1 * py[o]));
     if (k >= 2) w[o] = w[o] + dt * (-(t1 * pz[o]));
+}
+
+// The end of the all-physical step in one launch over k = 0..nz and all ld
+// columns: dpdz (k_dpdz), RHS - grad p (k_rhs_gradp), the projection
+// (k_project) with its boundary rows, and the constant planes of u, v, w, dpdx
+// and dpdy.  Each point reads and writes its own values, but for p
+// of the level below and the lid's u, v, which the level under it writes.
+// Bound by launches on small grids, where the eight it replaces took 4 to 5 us
+// each (96 x 48 x 64 mixed); one pass over each field instead of up to three on large ones.
+template <typename T>
+struct TailArgs {
+    T *u, *v, *w, *rx, *ry, *rz, *px, *py, *pz;
+    const T* p;
+    T dt, t1, dz, bogus;
+    const double* clk;
+};
+
+template <typename T>
+__global__ void k_press_tail(TailArgs<T> a, Geo g) {
+    int m, k, j, i;
+    long mb;
+    if (!pt_of(g, g.ld, m, k, j, i, mb)) return;
+    const long o = mb + (long)k * g.plane + (long)j * g.ld + i;
+    if (k == 0) {
+        a.u[o] = a.v[o] = a.w[o] = a.bogus;
+        return;
+    }
+    T pz;
+    if (i < g.nx) {
+        pz = (a.p[o] - a.p[o - g.plane]) / a.dz;
+        a.pz[o] = pz;
+    } else {
+        pz = a.pz[o];
+    }
+    a.rz[o] = a.rz[o] - pz;
+    if (k == g.nz) {
+        a.px[o] = a.py[o] = a.bogus;
+        a.w[o] = (T)0;
+        return;
+    }
+    const T px = a.px[o], py = a.py[o];
+    a.rx[o] = a.rx[o] - px;
+    a.ry[o] = a.ry[o] - py;
+    T u = a.u[o], v = a.v[o];
+    if (i < g.nx) {
+        T dt = a.dt, t1 = a.t1;
+        if (a.clk) {
+            dt = (T)a.clk[(long)CK_N * m + CK_DT];
+            t1 = (T)a.clk[(long)CK_N * m + CK_TADV1];
+        }
+        u = u + dt * (-(t1 * px));
+        v = v + dt * (-(t1 * py));
+        a.u[o] = u;
+        a.v[o] = v;
+        if (k >= 2) a.w[o] = a.w[o] + dt * (-(t1 * pz));
+    }
+    if (k == 1) a.w[o] = (T)0;
+    if (k == g.nz - 1) {
+        a.u[o + g.plane] = u;
+        a.v[o + g.plane] = v;
+    }
 }
 
 // Block-partial sums for the diagnostics (rmsdiv.f90:39-50, io.f90:115-124),
