@@ -21,9 +21,9 @@
 // projection and boundary kernels it replaces moved 21 + 4 (and the FP64
 // Thomas scratch) + 13 and ran the tridiagonal with one thread per column, a
 // chain of 2 nz divisions on half the chip's SIMDs.  Measured, those four
-// kernels and this one: 256 x 256 x 192 FP32 454 -> 312 us (3.7 TB/s), FP64
-// 826 -> 566 us (4.1 TB/s); 128^3 FP32 128 -> 45 us; 64^3 FP32 52 -> 14 us;
-// 32^3 FP64 34 -> 9.4 us.  What holds the largest back is address
+// kernels and this one: 256 x 256 x 192 FP32 454 -> 291 us (4.0 TB/s), FP64
+// 826 -> 540 us (4.3 TB/s); 128^3 FP32 128 -> 45 to 50 us; 64^3 FP32 52 -> 14
+// us; 32^3 FP64 34 -> 9.0 us.  What holds the largest back is address
 // translation: a thread's levels lie a plane apart in every array, so nearly
 // every line of a level misses the CU's first-level TLB (4.9 M misses for 5.3 M
 // lines with 128 bytes a row of the tile, 2.2 M with 256).
