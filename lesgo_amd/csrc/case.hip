@@ -1720,7 +1720,8 @@ void Case<T>::after_body() {
         // (nor the z derivatives)
         if (lag_now) stale &= ~(unsigned)(SG_SIJ | SG_DDZ);
         else stale |= SG_SIJ | SG_DDZ;
-        std::fill(mcold.begin(), mcold.end(), 0);
+        // (a member that is not stepped keeps its flag)
+        std::fill(mcold.begin(), mcold.begin() + Ma, 0);
     }
     if (st.on) stats_after_step();
 }

@@ -1,0 +1,41 @@
+"""Members of a batch that are not stepped (lg_set_active): one seeded while
+the others run starts from its own fields when it joins, to the bit.  No dynamic-model update and no disks."""
+import numpy as np
+import pytest
+
+import lesgo_amd
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = ("u", "v", "w", "p", "RHSx", "RHSz", "dudz", "dvdz", "txz", "tyz", "tzz")
+
+
+def cfg_of(precision="fp64", cfl=False):
+    return lesgo_amd.Config(24, 16, 9, dt=1e-5, precision=precision, initu=False, dyn_init=100,
+                            use_cfl_dt=cfl, cfl=0.05)
+
+
+def fields(c, member):
+    return {n: c.download(n, member=member) for n in FIELDS}
+
+
+def assert_same(a, b):
+    for n in a:
+        assert np.array_equal(a[n], b[n]), n
+
+
+@pytest.mark.parametrize("before", [1, 2])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_member_seeded_while_inactive_joins(precision, before):
+    with lesgo_amd.Case(cfg_of(precision)) as a:
+        a.seed_state(9, 0.1)
+        a.step(3)
+        want = fields(a, 0)
+    with lesgo_amd.Case(cfg_of(precision), members=2) as b:
+        b.set_active(1)
+        b.seed_state(5, 0.1)
+        b.seed_state(9, 0.1, member=1)
+        b.step(before)
+        b.set_active(2)
+        b.step_graph(3)
+        assert_same(want, fields(b, 1))
