@@ -862,11 +862,14 @@ void Case<T>::ddz_uvw() {
 // The planes whose values a step does not compute: BOGUS at the ghost level
 // and where the reference leaves it (derivatives.f90:214-311,
 // sgs_stag_util.f90:33-464), the lid's stresses and derivatives zero
-// (wallstress.f90:21-257, ubc_mom = 0).  Nothing but the host writes them, so a
-// spectral-resident case sets them on the steps that start from physical
-// fields only, in both buffers of the exchanged stresses and for every
-// member; the all-physical step at its head (one launch a step instead of
-// three: 32^3 FP64 2.6 us a launch, 256 x 256 x 192 4.8 us).
+// (wallstress.f90:21-257, ubc_mom = 0), and the wall level of dudz, dvdz, of
+// which the wall model then writes all but the padding columns.  Nothing else
+// of a step writes them, so a spectral-resident case sets them on the steps
+// that start from physical fields only, in both buffers of the exchanged
+// stresses; the all-physical step at its head (one launch a step instead of
+// three: 32^3 FP64 2.6 us a launch, 256 x 256 x 192 4.8 us).  Stepped members
+// only: the others' fields are theirs, and one that joins starts from its
+// physical fields or is copied with its planes.
 template <typename T>
 void Case<T>::fill_const_planes() {
     const int nz = d.nz;
@@ -900,7 +903,7 @@ void Case<T>::fill_const_planes() {
     static_assert(26 <= MAX_FILLS, "fill_const_planes needs more entries");
     a.mstride = d.field;
     a.plane = d.plane;
-    hipLaunchKernelGGL(k_fill_list<T>, dim3((unsigned)((d.plane + BLK - 1) / BLK), M, n),
+    hipLaunchKernelGGL(k_fill_list<T>, dim3((unsigned)((d.plane + BLK - 1) / BLK), Ma, n),
                        dim3(BLK), 0, stream, a);
 }
 

@@ -1,5 +1,6 @@
 """Members of a batch that are not stepped (lg_set_active): one seeded while
-the others run starts from its own fields when it joins, to the bit.  No dynamic-model update and no disks."""
+the others run starts from its own fields when it joins, and one that is
+parked keeps its fields, to the bit.  No dynamic-model update and no disks."""
 import numpy as np
 import pytest
 
@@ -39,3 +40,20 @@ def test_member_seeded_while_inactive_joins(precision, before):
         b.set_active(2)
         b.step_graph(3)
         assert_same(want, fields(b, 1))
+
+
+@pytest.mark.parametrize("cfl", [False, True])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_parked_member_keeps_its_fields(precision, cfl):
+    """Member 0 starts anew (from physical fields) and steps on while member 1
+    is parked."""
+    with lesgo_amd.Case(cfg_of(precision, cfl), members=2) as c:
+        for m in range(2):
+            c.seed_state(3 + m, 0.1, member=m)
+        c.set_counters(0, 0)
+        c.step(2)
+        c.set_active(1)
+        want = fields(c, 1)
+        c.seed_state(8, 0.1, member=0)
+        c.step(2)
+        assert_same(want, fields(c, 1))
