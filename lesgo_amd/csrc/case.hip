@@ -788,8 +788,8 @@ void Case<T>::filt_da(int f, int dfdx, int dfdy, cplx<T>* keep) {
 // (into tmp[0], tmp[1], level 0) ride with the inverses as jobs of one plane:
 // the G_test band of the same spectra (the reference's filtered plane to
 // rounding: G_test is 1/(nx ny) inside a sharp band and zero outside it and on
-// the Nyquist row; the band mask also drops the kx Nyquist column, which the
-// physical u, v do not carry).  A column launch of their own took 4 us.
+// the Nyquist row; the kx Nyquist column, which it zeroes too, is not stored).
+// A column launch of their own took 4 us.
 template <typename T>
 void Case<T>::filt_da_uvw(bool forward) {
     const T sc = (T)(1.0 / (d.nx * d.ny));

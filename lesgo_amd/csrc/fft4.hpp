@@ -147,8 +147,7 @@ __device__ __forceinline__ void cols_inv_load(cplx<T> (&x)[N1], const cplx<T>* s
                 const T g = gv[n1];
                 v = cplx<T>{g * v.x, g * v.y};
             } else if constexpr (K == K_GB) {
-                const bool in = gv[n1] != (T)0 && c != a.ncols - 1;
-                if (!in) v = cplx<T>{(T)0, (T)0};
+                if (gv[n1] == (T)0) v = cplx<T>{(T)0, (T)0};
             }
             (void)j;
             (void)nyq;
