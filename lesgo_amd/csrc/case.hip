@@ -189,7 +189,7 @@ Case<T>::Case(const lg_params& p, int members) : d(p), M(members), Ma(members) {
         // the spectra in one allocation: a thread of the column pass reads all
         // of them level by level, and fewer address translations miss when
         // they lie together (256 x 256 x 192 FP32: 286 against 300 us apart)
-        spool = dalloc<cplx<T>>((NSPEC + 3 + (spec_on ? 12 : 0)) * M * msp);
+        spool = dalloc<cplx<T>>((NSPEC + 3 + (spec_on ? 11 : 0)) * M * msp);
         cplx<T>* q = spool;
         auto take = [&] {
             cplx<T>* r = q;
@@ -206,7 +206,6 @@ Case<T>::Case(const lg_params& p, int members) : d(p), M(members), Ma(members) {
             for (int i = 0; i < 3; ++i) sF[i] = take();
             sP = take();
             sPf = take();
-            sDz = take();
         }
     }
     prod_fused = prod_fused_for(d.nx2, d.ny2, (int)sizeof(T));
@@ -223,7 +222,6 @@ Case<T>::Case(const lg_params& p, int members) : d(p), M(members), Ma(members) {
         hipLaunchKernelGGL(k_tridag_gam, dim3((n + 255) / 256), dim3(256), 0, stream, gam, tg);
         LG_HIP(hipGetLastError());
     }
-    usc = dalloc<double2>(M * msp);
     dev_err = dalloc<int>(1);
     lag_chunk = std::min(d.nz, 64);
     lag_fused = lag_fused_for(d.nx, d.ny, (int)sizeof(T));
@@ -310,7 +308,6 @@ Case<T>::~Case() {
     for (auto p : bigspec) fr(p);
     for (auto p : tmp) fr(p);
     fr(gam);
-    fr(usc);
     fr(dev_err);
     fr(lag_phys);
     fr(lag_spec);
@@ -474,13 +471,13 @@ size_t case_bytes(const lg_params& p, int members, int tsize) {
     b += (size_t)(12 + 3) * M * msp * 2 * T;                     // spec, sU/sV/sW
     const size_t nbig = prod_fused_for(d.nx2, d.ny2, tsize) ? 6 : 9;
     b += nbig * M * mbp * T + 6 * M * mbsp * 2 * T;              // big, bigspec
-    b += msp * sizeof(double) + M * msp * sizeof(double2);       // gam table, usc
+    b += msp * sizeof(double);                                   // gam table
     const bool lf = lag_fused_for(d.nx, d.ny, tsize);
     b += ((lf ? 0 : 15) + lag_filt_slots(lf, tsize)) * M * chunk * d.plane * T +
          21 * M * chunk * d.splane * 2 * T;
     b += 3 * M * sizeof(double) + 1024 * sizeof(double) + 2 * d.splane * T;
     b += M * (CK_N * sizeof(double) + 3 * sizeof(unsigned long long) + 2 * sizeof(int));
-    if (!p.use_cfl_dt) b += 12 * M * msp * 2 * T + 6 * M * d.field * T;   // spectral state
+    if (!p.use_cfl_dt) b += 11 * M * msp * 2 * T + 6 * M * d.field * T;   // spectral state
     return b;
 }
 
@@ -1383,7 +1380,8 @@ void Case<T>::press_stag_array(bool dpdz) {
         LG_LAUNCH(k_tridag<T>, dim3((nsys + tb - 1) / tb), dim3(tb), 0, stream,
                            (const cplx<T>*)spec[0], (const cplx<T>*)spec[1],
                            (const cplx<T>*)spec[2], (const cplx<T>*)spec[3],
-                           (const cplx<T>*)(spec[3] + d.splane), spec[4], gam, usc, tg, dev_err);
+                           (const cplx<T>*)(spec[3] + d.splane), spec[4], gam, tri_scratch(6), tg,
+                           dev_err);
     });
     {
         const cplx<T>* is[1] = {spec[4]};
@@ -1568,7 +1566,8 @@ void Case<T>::divstress_spec(cplx<T>* const* dwall) {
 // advection in spec[0..2], stresses in spec[6..11], u, v, w in sU, sV, sW;
 // p_hat into sP.  One launch (k_column) where the grid has a plan for it, else
 // the separate kernels (k_tridag scales u*, v*, w* by 1/(tadv1 dt) and takes
-// the divtz spectra of levels 1 and nz from sDz).
+// the divtz spectra of levels 1 and nz from a.dvz_bc, spec[5]; its scratch is
+// spec[3..4]: convec has finished with them).
 template <typename T>
 void Case<T>::column_spec(const SpecAb2<T>& a) {
     TriGeo tg{d.ny, d.NK, d.nz, d.splane, msp, Ma, 2.0 * PI_D / d.prm.lx,
@@ -1593,8 +1592,9 @@ void Case<T>::column_spec(const SpecAb2<T>& a) {
     timer.run(stream, KK_TRIDAG, tbytes, [&] {
         LG_LAUNCH(k_tridag<T>, dim3((nsys + tb - 1) / tb), dim3(tb), 0, stream,
                   (const cplx<T>*)sU, (const cplx<T>*)sV, (const cplx<T>*)sW,
-                  (const cplx<T>*)(sDz + d.splane), (const cplx<T>*)(sDz + d.nz * d.splane),
-                  sP, gam, usc, tg, dev_err);
+                  (const cplx<T>*)(a.dvz_bc + d.splane),
+                  (const cplx<T>*)(a.dvz_bc + d.nz * d.splane), sP, gam, tri_scratch(3), tg,
+                  dev_err);
     });
     hipLaunchKernelGGL(k_spec_project<T>, gs, dim3(BLK), 0, stream, (const cplx<T>*)sP, sU,
                        sV, sW, g, (T)d.prm.dt, (T)d.tadv1, (T)d.dz);
@@ -1662,8 +1662,8 @@ void Case<T>::step_body_spec(bool cold) {
         fwd2d(3, fs, scs, d.plane, kf0, d.field, sF, d.splane, kf0, msp, kf1 - kf0 + 1);
     }
     SpecAb2<T> a{spec[0], spec[1], spec[2],
-                 StressSpec<T>{spec[6], spec[7], spec[8], spec[9], spec[10], spec[11]}, sDz,
-                 (T)(1.0 / d.dz),
+                 StressSpec<T>{spec[6], spec[7], spec[8], spec[9], spec[10], spec[11]},
+                 spec[5], (T)(1.0 / d.dz),
                  tb ? sF[0] : nullptr, tb ? sF[1] : nullptr, tb ? sF[2] : nullptr,
                  sR[0], sR[1], sR[2], sRf[0], sRf[1], sRf[2], sPf, sU, sV, sW, d_mpf,
                  (const int*)d_flags, d.prm.use_mean_p_force, kf0, kf1,

@@ -153,7 +153,6 @@ struct Case {
     cplx<T>* sRf[3] = {};            // RHS_f spectra, alike
     cplx<T>* sP = nullptr;           // pressure spectrum of RHS's step, levels 0..nz
     cplx<T>* sPf = nullptr;          // of RHS_f's (zero where RHS_f holds - grad p already)
-    cplx<T>* sDz = nullptr;          // divtz spectra of the step (levels 1 and nz only)
     cplx<T>* sF[3] = {};             // forcing spectra of the step (disk levels)
     T* fprev[3] = {};                // the previous step's fxa, fya, fza
     T* tprev[3] = {};                // the previous step's txz, tyz, tzz
@@ -173,7 +172,7 @@ struct Case {
     T* fld[LG_NFIELDS] = {};
     // spectral scratch, each (nz+1) small spectral planes
     static constexpr int NSPEC = 12;
-    cplx<T>* spool = nullptr;        // every spectrum of the case (spec, sU ... sDz)
+    cplx<T>* spool = nullptr;        // every spectrum of the case (spec, sU ... sPf)
     cplx<T>* spec[NSPEC] = {};
     // big-grid scratch (levels 0..nz)
     static constexpr int NBIG = 9;
@@ -187,7 +186,6 @@ struct Case {
     cplx<T>* sV = nullptr;
     cplx<T>* sW = nullptr;
     double* gam = nullptr;           // (nz+1) * ny * NK: the pressure systems' gam table
-    double2* usc = nullptr;          // (nz+1) * ny * NK
     int* dev_err = nullptr;
     // Lagrangian model scratch (chunked over levels)
     int lag_chunk = 0;
@@ -279,6 +277,9 @@ struct Case {
     void after_body();
     void divstress_spec(cplx<T>* const* dwall);
     void column_spec(const SpecAb2<T>& a);
+    // k_tridag's FP64 scratch, (nz+1) * ny * NK per member, in spec[i] (a mixed
+    // case: spec[i] and spec[i + 1], which lie together)
+    double2* tri_scratch(int i) { return reinterpret_cast<double2*>(spec[i]); }
     void materialize(unsigned groups);
     void touch(bool modify);
     void high_part(T* const* f, T* const* out, int nf, int ka, int kb);

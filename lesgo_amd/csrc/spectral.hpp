@@ -135,7 +135,8 @@ __device__ __forceinline__ cplx<T> divt_z(const StressSpec<T>& t, long o, long S
 // u* = u + dt (t1 R + t2 (R_f - grad p_f)) in place of u (x, y on 1..nz-1,
 // z on 1..nz); members with euler[m] take R_f = R, p_f = 0.
 // divt is formed here from the stress spectra; its z component at levels 1
-// and nz (the pressure solve's boundary rows) is also stored in dvz_bc.
+// and nz (the pressure solve's boundary rows) is also stored in dvz_bc (any
+// scratch volume).
 template <typename T>
 struct SpecAb2 {
     const cplx<T> *cx, *cy, *cz;       // advection spectra

@@ -129,8 +129,8 @@ PassChoice pick(int kind, int N, int other, hipStream_t s, int reps, F&& trial) 
 }  // namespace
 
 // Tune every pass of c's step; returns the number of passes tuned.  Trials
-// write only scratch arrays (tmp, spec, big, bigspec, usc and the
-// spectra of the pressure solve), never the case's fields.
+// write only scratch arrays (tmp, spec, big, bigspec), never the case's
+// fields.
 template <typename T>
 int autotune(Case<T>& c, int reps) {
     const Dims& d = c.d;
@@ -219,8 +219,8 @@ int autotune(Case<T>& c, int reps) {
             hipLaunchKernelGGL(k_tridag<T>, dim3((nsys + tb - 1) / tb), dim3(tb), 0, s,
                                (const cplx<T>*)c.spec[0], (const cplx<T>*)c.spec[0],
                                (const cplx<T>*)c.spec[0], (const cplx<T>*)c.spec[0],
-                               (const cplx<T>*)(c.spec[0] + d.splane), c.spec[4], c.gam, c.usc,
-                               tg, c.dev_err);
+                               (const cplx<T>*)(c.spec[0] + d.splane), c.spec[4], c.gam,
+                               c.tri_scratch(6), tg, c.dev_err);
         });
         ++n;
     }
