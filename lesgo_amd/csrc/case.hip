@@ -185,6 +185,8 @@ Case<T>::Case(const lg_params& p, int members) : d(p), M(members), Ma(members) {
     // environment keeps every case on the all-physical step
     const char* phys = std::getenv("LESGO_AMD_PHYSICAL_STEP");
     spec_on = !cfl_mode && !(phys && phys[0] == '1');
+    const char* col = std::getenv("LESGO_AMD_COLUMN");
+    col_fused = column_plan<T>(d.nz, d.ny * d.NK, d.splane).L && !(col && col[0] == '0');
     {
         // the spectra in one allocation: a thread of the column pass reads all
         // of them level by level, and fewer address translations miss when
@@ -1373,7 +1375,8 @@ void Case<T>::press_stag_array(bool dpdz) {
         (double)Ma * d.splane * sizeof(cplx<T>) * (3.0 * d.nz + 1 + 2 + d.nz + 1);
     timer.run(stream, KK_TRIDAG, tbytes, [&] {
         const ColPress<T> cp{spec[0], spec[1], spec[2], spec[3], spec[3] + d.splane};
-        if (launch_column<T, false>(SpecAb2<T>{}, cp, spec_geo<T>(d, msp, 1, d.nz), tg, spec[4],
+        if (col_fused &&
+            launch_column<T, false>(SpecAb2<T>{}, cp, spec_geo<T>(d, msp, 1, d.nz), tg, spec[4],
                                     gam, (T)d.dz, dev_err, Ma, stream))
             return;
         const int nsys = Ma * d.ny * d.NK, tb = choice_for<T>(PK_TRIDAG, d.ny, d.NK).S;
@@ -1574,14 +1577,16 @@ void Case<T>::column_spec(const SpecAb2<T>& a) {
               2.0 * PI_D / d.prm.ly, d.dz, 1.0 / (d.dz * d.dz), 1.0 / d.dz};
     tg.hsc = (1.0 / d.tadv1) / d.prm.dt;
     const SpecGeo<T> g = spec_geo<T>(d, msp, 1, d.nz);
-    if (column_plan<T>(d.nz, d.ny * d.NK, d.splane).L) {
+    if (col_fused) {
         // sixteen spectra in and seven out, and the forcing on its levels
         const double cb = (double)Ma * d.splane * sizeof(cplx<T>) *
                           (23.0 * d.nz + (a.fx ? 3.0 * (a.kf1 - a.kf0 + 1) : 0.0));
+        bool done = false;
         timer.run(stream, KK_TRIDAG, cb, [&] {
-            launch_column<T, true>(a, ColPress<T>{}, g, tg, sP, gam, (T)d.dz, dev_err, Ma, stream);
+            done = launch_column<T, true>(a, ColPress<T>{}, g, tg, sP, gam, (T)d.dz, dev_err, Ma,
+                                          stream);
         });
-        return;
+        if (done) return;
     }
     const int n = d.ny * d.NK;
     const dim3 gs((n + BLK - 1) / BLK, d.nz * Ma);

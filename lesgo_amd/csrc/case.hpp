@@ -137,6 +137,10 @@ struct Case {
     // (k_rows_r2c_prod) where that length has a four-step split;
     // LESGO_AMD_PROD_ROWS=0 keeps k_products and the three product fields
     bool prod_fused = true;
+    // the spectra's AB2 update, pressure solve and projection run in one kernel
+    // (k_column) where the grid has a plan for it; LESGO_AMD_COLUMN=0 keeps
+    // the separate kernels
+    bool col_fused = true;
     std::vector<char> mcold;
     // members whose last step started from their physical fields (their
     // RHS_f high part is in the physical RHS_f only); the others take it
