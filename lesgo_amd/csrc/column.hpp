@@ -42,14 +42,13 @@ struct ColPress {
     const cplx<T> *rb, *rt;            // Neumann planes, bottom and top
 };
 
-// LDS of a block of nthr threads: the u* slots (STEP) and, per wave and
-// column, a chunk total (value and factor; the neighbour levels share its
-// place); row 0.
+// LDS of a block of nthr threads: row 0 and the solution passed from wave to
+// wave (one value per column each), the levels that waves hand to their
+// neighbours (one per wave and column) and the u* slots (STEP).
 template <typename T>
 constexpr size_t column_lds(int L, int CT, int nthr, bool step) {
-    return (size_t)nthr * (step ? 3 * L * sizeof(cplx<T>) : 0) +
-           (size_t)(nthr / 64) * CT * (sizeof(double2) + sizeof(double)) +
-           (size_t)CT * sizeof(double2);
+    return (size_t)2 * CT * sizeof(double2) + (size_t)(nthr / 64) * CT * sizeof(cplx<T>) +
+           (size_t)nthr * (step ? 3 * L * sizeof(cplx<T>) : 0);
 }
 
 template <typename T>
@@ -80,11 +79,10 @@ __global__ void __launch_bounds__(column_max_threads<T>(), sizeof(T) == 4 ? 4 : 
     const int nthr = blockDim.x;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6, NW = nthr >> 6;
-    double2* xe = reinterpret_cast<double2*>(smem_col);          // [wave][CT] totals
-    double2* x0 = xe + NW * CT;                                  // [CT] row 0
-    double* xf = reinterpret_cast<double*>(x0 + CT);             // [wave][CT] factors
-    cplx<T>* xn = reinterpret_cast<cplx<T>*>(xe);                // [wave][CT] neighbour level
-    cplx<T>* Ul = reinterpret_cast<cplx<T>*>(xf + NW * CT);      // [3 L][threads] u*
+    double2* x0 = reinterpret_cast<double2*>(smem_col);          // [CT] row 0
+    double2* xe = x0 + CT;                                       // [CT] a wave's last value
+    cplx<T>* xn = reinterpret_cast<cplx<T>*>(xe + CT);           // [wave][CT] neighbour level
+    cplx<T>* Ul = xn + NW * CT;                                  // [3 L][threads] u*
     const int zc = tid / CT, c0 = tid - zc * CT;
     const bool wlo = lane < CT, whi = lane >= 64 - CT;           // a wave's end chunks
     const int ncol = g.ny * g.NK;
@@ -246,8 +244,13 @@ __global__ void __launch_bounds__(column_max_threads<T>(), sizeof(T) == 4 ? 4 : 
         // 1e-16 roundings visible at 1e-8 within some 100 steps).  The chain is
         // short: the pivots and their reciprocals are formed by every chunk at
         // once, and a quotient t / bet is q = t rb corrected by its remainder,
-        // fma(fma(-q, bet, t), rb, q), the correctly rounded one (Markstein) as
-        // rb = 1 / bet is.
+        // fma(fma(-q, bet, t), rb, q) (Markstein).  With rb = 1 / bet correctly
+        // rounded q is within 1.5 ulp and the result is t / bet rounded unless
+        // t / bet lies within some 2^-52 ulp of the middle between two doubles;
+        // below about 1e-290 the remainder underflows and the result is the
+        // uncorrected q, and an infinite t gives NaN where a division gives
+        // infinity (a run that has diverged).  tests/test_gpu_column_bits.py
+        // compares whole steps with k_tridag's divisions.
         const double c3 = tg.const3;
         const double b_in = -(kxd * kxd + kyd * kyd + 2.0 * c3);
         auto quot = [](double t, double bet, double rb) {

@@ -42,7 +42,7 @@ def assert_same(a, b, members, what):
 GRIDS = {
     "fp64": [(8, 8, 3), (12, 8, 16), (16, 8, 63), (8, 8, 128), (8, 8, 250), (64, 72, 55),
              (64, 64, 100), (64, 64, 192)],
-    "mixed": [(8, 8, 3), (16, 8, 31), (8, 8, 48), (8, 8, 96), (8, 8, 224), (8, 8, 390),
+    "mixed": [(8, 8, 3), (16, 8, 31), (8, 8, 48), (8, 8, 96), (8, 8, 224), (8, 8, 390), (8, 8, 410),
               (96, 96, 33), (128, 64, 64), (128, 64, 81), (128, 64, 150)],
 }
 
