@@ -512,11 +512,11 @@ template <typename T>
 void Case<T>::fwd2d(int njobs, const T* const* src, const T* scales, long src_plane, int src_lev0,
                     long src_ms, cplx<T>* const* dst, long dst_plane, int dst_lev0, long dst_ms,
                     int nlev, const double* mscale, int band_nzc, int band_ykeep,
-                    const int* nl) {
+                    int nride, int nlr) {
     if (nlev <= 0) return;
     launch_rows_r2c<T>(timer, px.plan, njobs, src, scales, src_plane, d.ld, src_lev0, src_ms, dst,
                        dst_plane, dst_lev0, dst_ms, d.ny, d.NK, nlev, Ma, stream, nullptr,
-                       mscale, CK_N, band_nzc, nl);
+                       mscale, CK_N, band_nzc, nride, nlr);
     for (int j0 = 0; j0 < njobs; j0 += MAX_JOBS) {
         const int nj = std::min(MAX_JOBS, njobs - j0);
         ColArgs<T> c{};
@@ -527,8 +527,9 @@ void Case<T>::fwd2d(int njobs, const T* const* src, const T* scales, long src_pl
             c.op[i] = OP_NONE;
             c.nzc[i] = band_nzc;
             c.ykeep[i] = band_ykeep;
-            c.nl[i] = nl ? nl[j0 + i] : 0;
         }
+        c.nfull = std::max(0, std::min(nj, njobs - nride - j0));
+        c.nlr = c.nfull < nj ? nlr : 0;
         c.src_plane = c.dst_plane = dst_plane;
         c.lev0_src = c.lev0_dst = dst_lev0;
         c.src_mstride = c.dst_mstride = dst_ms;
@@ -543,7 +544,7 @@ template <typename T>
 void Case<T>::inv2d(int njobs, const cplx<T>* const* src, const int* ops, long src_plane,
                     int src_lev0, long src_ms, T* const* dst, long dst_plane, int dst_lev0,
                     long dst_ms, int nlev, cplx<T>* const* tmpspec, const cplx<T>* const* src2,
-                    const int* nl) {
+                    int nride, int nlr) {
     if (nlev <= 0) return;
     // column-pass output goes to tmpspec[i], planes 0..nlev-1, members packed
     const long tms = (long)nlev * d.splane;
@@ -559,7 +560,8 @@ void Case<T>::inv2d(int njobs, const cplx<T>* const* src, const int* ops, long s
         bool taken[MAX_JOBS] = {};
         T* rdst[MAX_JOBS] = {};
         T* rdst2[MAX_JOBS] = {};
-        int nce[MAX_JOBS] = {}, rnl[MAX_JOBS] = {};
+        int nce[MAX_JOBS] = {};
+        int nf = 0;          // jobs of every plane, before the riding ones
         for (int i = 0; i < nj; ++i) {
             if (taken[i]) continue;
             c.src[nc] = src[j0 + i];
@@ -567,7 +569,7 @@ void Case<T>::inv2d(int njobs, const cplx<T>* const* src, const int* ops, long s
             c.dst[nc] = tmpspec[nc];
             c.op[nc] = ops[j0 + i];
             rdst[nc] = dst[j0 + i];
-            c.nl[nc] = rnl[nc] = nl ? nl[j0 + i] : 0;
+            if (j0 + i < njobs - nride) nf = nc + 1;
             const bool g1 = ops[j0 + i] == OP_G1 || ops[j0 + i] == OP_G1B;
             nce[nc] = g1 ? g_nzc[0] : ops[j0 + i] == OP_G2 ? g_nzc[1] : 0;
             if (g1 || ops[j0 + i] == OP_G2) {
@@ -598,18 +600,18 @@ void Case<T>::inv2d(int njobs, const cplx<T>* const* src, const int* ops, long s
         c.map = MAP_ID;
         c.zero_nyq = 0;
         col_common(c, d, G1, G2);
+        c.nfull = nf;
+        c.nlr = nf < nc ? nlr : 0;
         launch_cols<T, +1>(timer, c, nc, nlev, Ma, d.ny, stream, nullptr);
         // the row pass: the jobs of every plane in one launch, then the ones of
         // a few planes that rode with them (last in the list), over their band
         std::vector<const cplx<T>*> ts(tmpspec, tmpspec + nc);
-        int nf = nc;
-        while (nf > 0 && rnl[nf - 1]) --nf;
         for (int f = 0; f < 2; ++f) {
             const int i0 = f ? nf : 0, n = f ? nc - nf : nf;
             if (n > 0)
                 launch_rows_c2r<T>(timer, px.plan, n, ts.data() + i0, d.splane, 0, tms, rdst + i0,
                                    dst_plane, d.ld, dst_lev0, dst_ms, d.ny, d.NK,
-                                   f ? rnl[nf] : nlev, Ma, stream, nullptr, nce + i0, rdst2 + i0,
+                                   f ? nlr : nlev, Ma, stream, nullptr, nce + i0, rdst2 + i0,
                                    (T)(2.0 * PI_D / d.prm.lx));
         }
     }
@@ -801,9 +803,9 @@ void Case<T>::filt_da_uvw(bool forward) {
                          OP_NONE, OP_IKX, OP_IKY, OP_G1B,  OP_G1B};
     T* dst[11] = {fld[LG_U],    fld[LG_DUDX], fld[LG_DUDY], fld[LG_V], fld[LG_DVDX], fld[LG_DVDY],
                   fld[LG_W],    fld[LG_DWDX], fld[LG_DWDY], tmp[0],    tmp[1]};
-    const int nl[11] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 1, 1};
-    inv2d(forward ? 9 : 11, is, ops, d.splane, 0, msp, dst, d.plane, 0, d.field, d.nz + 1, spec,
-          nullptr, nl);
+    const int nride = forward ? 0 : 2;
+    inv2d(9 + nride, is, ops, d.splane, 0, msp, dst, d.plane, 0, d.field, d.nz + 1, spec,
+          nullptr, nride, 1);
 }
 
 template <typename T>
@@ -1561,8 +1563,7 @@ void Case<T>::divstress_spec(cplx<T>* const* dwall) {
     const T scs[8] = {sc, sc, sc, sc, sc, sc, sc, sc};
     cplx<T>* S[8] = {spec[6], spec[7],  spec[8],  spec[9],
                      spec[10], spec[11], dwall[0] - d.splane, dwall[1] - d.splane};
-    const int nl[8] = {0, 0, 0, 0, 0, 0, 1, 1};
-    fwd2d(8, src, scs, d.plane, 1, d.field, S, d.splane, 1, msp, d.nz, nullptr, 0, 0, nl);
+    fwd2d(8, src, scs, d.plane, 1, d.field, S, d.splane, 1, msp, d.nz, nullptr, 0, 0, 2, 1);
 }
 
 // The AB2 update, the pressure solve and the projection on the spectra:

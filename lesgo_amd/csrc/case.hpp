@@ -219,16 +219,17 @@ struct Case {
     T* mem(int id, int m) { return fld[id] + (long)m * d.field; }
 
     // 2-D transform helpers over planes [lev0, lev0+nlev) of every member
-    // nl: planes of each job (null or 0: nlev); band (nzc, ykeep; 0: none): the spectra are only read inside the test
-    // filters' band, so only that part is computed and written
+    // the last nride jobs have nlr planes, the others nlev; band (nzc, ykeep;
+    // 0: none): the spectra are only read inside the test filters' band, so
+    // only that part is computed and written
     void fwd2d(int njobs, const T* const* src, const T* scales, long src_plane, int src_lev0,
                long src_ms, cplx<T>* const* dst, long dst_plane, int dst_lev0, long dst_ms,
                int nlev, const double* mscale = nullptr, int band_nzc = 0, int band_ykeep = 0,
-               const int* nl = nullptr);
+               int nride = 0, int nlr = 0);
     void inv2d(int njobs, const cplx<T>* const* src, const int* ops, long src_plane, int src_lev0,
                long src_ms, T* const* dst, long dst_plane, int dst_lev0, long dst_ms, int nlev,
                cplx<T>* const* tmpspec, const cplx<T>* const* src2 = nullptr,
-               const int* nl = nullptr);
+               int nride = 0, int nlr = 0);
     void pad_inv_big(int njobs, const cplx<T>* const* src, int lev0, int nlev);
     void fwd_big_unpad(int njobs, const T* const* src, cplx<T>* const* dst, int lev0, int nlev);
     void cols_unpad(int njobs, cplx<T>* const* dst, int lev0, int nlev);

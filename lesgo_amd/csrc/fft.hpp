@@ -231,11 +231,9 @@ struct RowR2CArgs {
     int mscale_stride;
     int nwr;               // columns of dst written (0: ncols; a band-limited consumer
                            // reads no more; the four-step and generic kernels honour it)
-    // a job of few planes rides with others in one launch (ride set): nl[job] is
-    // its number of planes (0: nlev), its blocks past them end at once.  Without
-    // riders no block waits for the indexed nl before its other loads.
-    int ride;
-    int nl[MAX_JOBS];
+    // jobs of few planes ride with others in one launch: the jobs from nfull on
+    // have nlr planes (0: none rides), their blocks past them end at once
+    int nfull, nlr;
 };
 
 // The fields the convective products are formed from (prod_rows.hpp): u, v,
@@ -255,7 +253,7 @@ __global__ void __launch_bounds__(256) k_rows_r2c(RowR2CArgs<T> a) {
     const int job = blockIdx.z;
     const int mem = blockIdx.y / a.nlev;
     const int plane = blockIdx.y - mem * a.nlev;
-    if (a.ride && a.nl[job] && plane >= a.nl[job]) return;
+    if (a.nlr && job >= a.nfull && plane >= a.nlr) return;
     const int npairs = a.nrows / 2;
     const int pair0 = blockIdx.x * a.S;
     const int S = min(a.S, npairs - pair0);
@@ -460,8 +458,7 @@ struct ColArgs {
     // inverse MAP_ID jobs: the input's ky = ny/2 row is taken as zero (as
     // filt_da's is) when set
     int nyq0[MAX_JOBS];
-    int ride;
-    int nl[MAX_JOBS];  // planes of the job (0: nlev), as RowR2CArgs
+    int nfull, nlr;    // riding jobs, as RowR2CArgs
 };
 
 // Row jb of a small-grid spectrum inside the band |m| < ykeep (0: all rows).
@@ -519,7 +516,7 @@ __global__ void __launch_bounds__(256) k_cols(ColArgs<T> a) {
     const int ykeep = a.ykeep[job];
     const int mem = blockIdx.z / a.nlev;
     const int plane = blockIdx.z - mem * a.nlev;
-    if (a.ride && a.nl[job] && plane >= a.nl[job]) return;
+    if (a.nlr && job >= a.nfull && plane >= a.nlr) return;
     const cplx<T>* src = a.src[job] + mem * a.src_mstride + (long)(a.lev0_src + plane) * a.src_plane;
     cplx<T>* dst = a.dst[job] + mem * a.dst_mstride + (long)(a.lev0_dst + plane) * a.dst_plane;
     const int op = a.op[job];

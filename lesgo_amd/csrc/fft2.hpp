@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(256) k_rows_r2c_v2(RowR2CArgs<T> a) {
     const int job = blockIdx.z;
     const int mem = blockIdx.y / a.nlev;
     const int plane = blockIdx.y - mem * a.nlev;
-    if (a.ride && a.nl[job] && plane >= a.nl[job]) return;
+    if (a.nlr && job >= a.nfull && plane >= a.nlr) return;
     const int npairs = a.nrows / 2;
     const int pair0 = blockIdx.x * a.S;
     const int S = min(a.S, npairs - pair0);
@@ -348,7 +348,7 @@ __global__ void __launch_bounds__(256) k_cols_v2(ColArgs<T> a) {
     const int ykeep = a.ykeep[job];
     const int mem = blockIdx.z / a.nlev;
     const int plane = blockIdx.z - mem * a.nlev;
-    if (a.ride && a.nl[job] && plane >= a.nl[job]) return;
+    if (a.nlr && job >= a.nfull && plane >= a.nlr) return;
     const cplx<T>* src = a.src[job] + mem * a.src_mstride + (long)(a.lev0_src + plane) * a.src_plane;
     cplx<T>* dst = a.dst[job] + mem * a.dst_mstride + (long)(a.lev0_dst + plane) * a.dst_plane;
     const int op = a.op[job];

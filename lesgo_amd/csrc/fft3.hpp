@@ -46,7 +46,7 @@ __global__ void __launch_bounds__(256) k_rows_r2c_v3(RowR2CArgs<T> a) {
     const int job = blockIdx.z;
     const int mem = blockIdx.y / a.nlev;
     const int plane = blockIdx.y - mem * a.nlev;
-    if (a.ride && a.nl[job] && plane >= a.nl[job]) return;
+    if (a.nlr && job >= a.nfull && plane >= a.nlr) return;
     const int npairs = a.nrows / 2;
     const int pair0 = blockIdx.x * a.S;
     const int S = min(a.S, npairs - pair0);

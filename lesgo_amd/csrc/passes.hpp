@@ -89,14 +89,15 @@ std::vector<std::pair<int, int>> pass_splits(int N);
 // spectra: r2c writes only columns < nwr (0: all), c2r reads only columns
 // < nce[job] (null or 0: all) and takes the rest as zero.  c2r jobs with
 // dst2[job] set also write the x derivative (i kx times the input, kxs =
-// 2 pi / Lx) there.  r2c: nl, planes of each job (null or 0: nlev).
+// 2 pi / Lx) there.  r2c: the last nride jobs have nlr
+// planes each, the others nlev.
 template <typename T>
 void launch_rows_r2c(KernelTimer& tm, const FftPlan& pl, int njobs, const T* const* src,
                      const T* scales, long src_plane, int src_ld, int src_lev0, long src_ms,
                      cplx<T>* const* dst, long dst_plane, int dst_lev0, long dst_ms, int nrows,
                      int ncols, int nlev, int M, hipStream_t s, const PassChoice* force,
                      const double* mscale = nullptr, int mscale_stride = 0, int nwr = 0,
-                     const int* nl = nullptr);
+                     int nride = 0, int nlr = 0);
 template <typename T>
 void launch_rows_c2r(KernelTimer& tm, const FftPlan& pl, int njobs, const cplx<T>* const* src,
                      long src_plane, int src_lev0, long src_ms, T* const* dst, long dst_plane,

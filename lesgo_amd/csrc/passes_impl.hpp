@@ -304,20 +304,20 @@ void launch_rows_r2c(KernelTimer& tm, const FftPlan& pl, int njobs, const T* con
                      const T* scales, long src_plane, int src_ld, int src_lev0, long src_ms,
                      cplx<T>* const* dst, long dst_plane, int dst_lev0, long dst_ms, int nrows,
                      int ncols, int nlev, int M, hipStream_t s, const PassChoice* force,
-                     const double* mscale, int mscale_stride, int nwr, const int* nl) {
+                     const double* mscale, int mscale_stride, int nwr, int nride, int nlr) {
     const PassChoice ch = force ? *force : choice_for<T>(PK_R2C, pl.N, nrows);
     for (int j0 = 0; j0 < njobs; j0 += MAX_JOBS) {
         const int nj = std::min(MAX_JOBS, njobs - j0);
         RowR2CArgs<T> a{};
         a.plan = pl;
-        double planes = 0.0;   // summed over the jobs
+        a.nfull = std::max(0, std::min(nj, njobs - nride - j0));
+        a.nlr = a.nfull < nj ? nlr : 0;
+        // summed over the jobs
+        const double planes = (double)a.nfull * nlev + (double)(nj - a.nfull) * nlr;
         for (int i = 0; i < nj; ++i) {
             a.src[i] = src[j0 + i];
             a.dst[i] = dst[j0 + i];
             a.scale[i] = scales ? scales[j0 + i] : (T)1;
-            a.nl[i] = nl ? nl[j0 + i] : 0;
-            a.ride |= a.nl[i];
-            planes += a.nl[i] ? a.nl[i] : nlev;
         }
         a.src_plane = src_plane;
         a.dst_plane = dst_plane;
@@ -418,18 +418,16 @@ void launch_cols(KernelTimer& tm, ColArgs<T>& c, int nj, int nlev, int M, int ny
     // band-limited jobs: columns < nzc, and (MAP_ID) rows |ky| < ykeep read by
     // an inverse pass or written by a forward one
     int cmax = 0;
-    c.ride = 0;
     double cols_rw = 0.0;      // sum over jobs of planes x columns x rows moved
     for (int i = 0; i < nj; ++i) {
         const int nzc = (c.nzc[i] > 0 && c.nzc[i] < c.ncols) ? c.nzc[i] : c.ncols;
         c.nzc[i] = nzc < c.ncols ? nzc : 0;
         cmax = std::max(cmax, nzc);
-        c.ride |= c.nl[i];
         const int band = c.ykeep[i] > 0 ? std::min(2 * c.ykeep[i] - 1, ny_in) : 0;
         const double rin = (DIR > 0 && band) ? band : ny_in;
         // MAP_UNPAD writes the small grid's ny rows, not the N it transforms
         const double rout = c.map == MAP_UNPAD ? c.ny : ((DIR < 0 && band) ? band : N);
-        cols_rw += (double)(c.nl[i] ? c.nl[i] : nlev) * nzc * (rin + rout);
+        cols_rw += (double)(c.nlr && i >= c.nfull ? c.nlr : nlev) * nzc * (rin + rout);
     }
     dim3 grid(nj, (cmax + c.TC - 1) / c.TC, nlev * M);
     const double bytes = (double)M * sizeof(cplx<T>) * cols_rw;
