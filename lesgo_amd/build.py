@@ -13,9 +13,14 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "liblesgo_amd.so")
-SOURCES = ["case.hip", "passes_f64.hip", "passes_f64_cols.hip", "passes_f64_fused.hip",
-           "passes_f32.hip", "passes_f32_cols.hip", "passes_f32_fused.hip", "tune.hip",
-           "turbines.hip", "capi.hip", "server.hip", "stats.hip", "calibrate.hip", "tridag.hip"]
+# One object per precision for the transform passes, though three would build
+# in 2.5 minutes instead of 4.5: a process's malloc keeps freed memory up to
+# twice the largest buffer it has mapped and freed, and the runtime's copy of
+# that code object is the one that counts.  With smaller objects four fields
+# of 2.5 MB read back and freed (96 x 48 x 64 FP64) are unmapped and faulted
+# in again each time: 1900 us the four instead of 610.
+SOURCES = ["case.hip", "passes_f64.hip", "passes_f32.hip", "tune.hip", "turbines.hip", "capi.hip",
+           "server.hip", "stats.hip", "calibrate.hip", "tridag.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

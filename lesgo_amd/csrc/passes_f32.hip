@@ -1,4 +1,4 @@
-// Launch choices and row-pass launchers instantiated for float.
+// Transform-pass launchers instantiated for float.
 #include "passes_impl.hpp"
 
 namespace lg {
@@ -14,4 +14,16 @@ template void launch_rows_c2r<float>(KernelTimer&, const FftPlan&, int, const cp
                                    long, int, long, float* const*, long, int, int, long, int, int,
                                    int, int, hipStream_t, const PassChoice*, const int*,
                                    float* const*, float);
+template void launch_cols<float, -1>(KernelTimer&, ColArgs<float>&, int, int, int, int, hipStream_t,
+                                   const PassChoice*);
+template void launch_cols<float, +1>(KernelTimer&, ColArgs<float>&, int, int, int, int, hipStream_t,
+                                   const PassChoice*);
+template bool launch_lag_rows<float>(KernelTimer&, const LagRowArgs<float>&, int, hipStream_t);
+template bool lag_rows_ok<float>(int, int);
+template bool launch_rows_r2c_prod<float>(KernelTimer&, const FftPlan&, const ProdSrc<float>&, long,
+                                          int, int, long, cplx<float>* const*, long, long, int,
+                                          int, int, int, hipStream_t);
+template bool prod_rows_ok<float>(int, int);
+template bool launch_lag_prep_rows<float>(KernelTimer&, const LagPrepArgs<float>&, int, hipStream_t);
+
 }  // namespace lg
