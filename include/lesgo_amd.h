@@ -256,7 +256,9 @@ int lg_calibrate_copy(long nbytes, int reps, double* ms_per_copy);
  * subsystems) or on member 0 (copies, seeding, diagnostics, disks).  Member
  * m's arithmetic is identical to the same case run alone. */
 int lg_create_batch(const lg_params* prm, int members, lg_case** out);
-/* Capacity and number of stepped members (members 0..active-1). */
+/* Capacity and number of stepped members (members 0..active-1).  A member
+ * that is not stepped keeps its fields and goes on from them when it is made
+ * active again. */
 int lg_batch_info(const lg_case* c, int* members, int* active);
 int lg_set_active(lg_case* c, int active);
 /* Per-member z0 (wallstress.f90:198) and mean_p_force (main.f90:228-232). */

@@ -91,8 +91,9 @@ bool smooth(int n) {
 void check_field(int id) { REQUIRE(id >= 0 && id < LG_NFIELDS, "field id out of range"); }
 
 template <typename C>
-void check_member(const C& c, int m) {
+void check_member(C& c, int m) {
     REQUIRE(m >= 0 && m < c.M, "member index out of range");
+    c.settle(m);
 }
 
 }  // namespace
@@ -512,7 +513,7 @@ int lg_batch_info(const lg_case* h, int* members, int* active) {
 int lg_set_active(lg_case* h, int active) {
     return dispatch_read(h, [&](auto& c) {
         REQUIRE(active >= 1 && active <= c.M, "active member count out of range");
-        c.Ma = active;
+        c.set_active(active);
     });
 }
 

@@ -244,6 +244,7 @@ Case<T>::Case(const lg_params& p, int members) : d(p), M(members), Ma(members) {
     dflags_now.assign(6 * M, 0);
     d_flags = dalloc<int>(6L * M);
     mcold.assign(M, 1);
+    mswapped.assign(M, 0);
     rhsf_phys.assign(M, 1);
     d_clock = dalloc<double>((long)CK_N * M);
     d_cmax = dalloc<unsigned long long>(3L * M);
@@ -389,6 +390,7 @@ void Case<T>::seed_member(int m, long seed, double noise) {
     lm_init[m] = 0;
     clock_reset(m);
     mcold[m] = 1;
+    mswapped[m] = swapped;
 }
 
 // ---------------------------------------------------------------------------
@@ -1686,6 +1688,7 @@ void Case<T>::swap_rhs() {
     std::swap(fld[LG_RHSY], fld[LG_RHSY_F]);
     std::swap(fld[LG_RHSZ], fld[LG_RHSZ_F]);
     swapped = !swapped;
+    std::fill(mswapped.begin(), mswapped.begin() + Ma, (char)swapped);
     if (!spec_on) return;
     for (int q = 0; q < 3; ++q) std::swap(sR[q], sRf[q]);
     std::swap(sP, sPf);
@@ -1706,6 +1709,46 @@ void Case<T>::swap_rhs() {
     if (fclear_pending > 0 && --fclear_pending == 0)
         for (int id : {LG_FXA, LG_FYA, LG_FZA})
             LG_HIP(hipMemsetAsync(fld[id], 0, M * d.field * sizeof(T), stream));
+}
+
+// A step exchanges the buffers of every member, stepped or not (swap_rhs).
+// Before a member that sat out an odd number of steps is read, written or
+// stepped again its own slices are put back where they belong.
+template <typename T>
+void Case<T>::settle(int m) {
+    if (mswapped[m] == (char)swapped) return;
+    mswapped[m] = swapped;
+    SwapList<T> f{}, s{};
+    int n = 0;
+    auto put = [&](T* a, T* b) {
+        f.a[n] = a + (long)m * d.field;
+        f.b[n++] = b + (long)m * d.field;
+    };
+    put(fld[LG_RHSX], fld[LG_RHSX_F]);
+    put(fld[LG_RHSY], fld[LG_RHSY_F]);
+    put(fld[LG_RHSZ], fld[LG_RHSZ_F]);
+    if (spec_on) {
+        const int fx[3] = {LG_FXA, LG_FYA, LG_FZA}, tz[3] = {LG_TXZ, LG_TYZ, LG_TZZ};
+        for (int q = 0; q < 3; ++q) put(fld[fx[q]], fprev[q]);
+        for (int q = 0; q < 3; ++q) put(fld[tz[q]], tprev[q]);
+        for (int q = 0; q < 4; ++q) {
+            s.a[q] = reinterpret_cast<T*>((q < 3 ? sR[q] : sP) + (long)m * msp);
+            s.b[q] = reinterpret_cast<T*>((q < 3 ? sRf[q] : sPf) + (long)m * msp);
+        }
+        s.n = 2 * msp;
+        hipLaunchKernelGGL(k_swap_list<T>, dim3((unsigned)((s.n + BLK - 1) / BLK), 4), dim3(BLK),
+                           0, stream, s);
+    }
+    f.n = d.field;
+    hipLaunchKernelGGL(k_swap_list<T>, dim3((unsigned)((f.n + BLK - 1) / BLK), n), dim3(BLK), 0,
+                       stream, f);
+    LG_HIP(hipGetLastError());
+}
+
+template <typename T>
+void Case<T>::set_active(int n) {
+    for (int m = Ma; m < n; ++m) settle(m);
+    Ma = n;
 }
 
 template <typename T>

@@ -94,6 +94,9 @@ struct Case {
     HostCopy hcopy;                  // staging of fields read back
     int jt = 0, jt_total = 0;
     bool swapped = false;            // RHS / RHS_f storage exchanged (odd steps)
+    // the value of `swapped` that a member's exchanged buffers lie by: for one
+    // that is not stepped, that of its last step (settle)
+    std::vector<char> mswapped;
     std::vector<double> zo, mpf;     // per member z0 and mean_p_force (x, y)
     double* d_denom = nullptr;       // per member ln(0.5 dz / z0)
     double* d_mpf = nullptr;         // per member mean_p_force_x, _y
@@ -276,6 +279,8 @@ struct Case {
     void step_body();
     void step_body_spec(bool cold);
     void swap_rhs();
+    void settle(int m);
+    void set_active(int n);
     int count_cold() const;
     void copy_spec_member(int src, int dst);
     void run_body(bool cold);

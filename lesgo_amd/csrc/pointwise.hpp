@@ -72,6 +72,25 @@ __global__ void k_copy_plane(const T* src, T* dst, long mstride, long n) {
     if (idx < n) dst[(long)blockIdx.y * mstride + idx] = src[(long)blockIdx.y * mstride + idx];
 }
 
+// Arrays of n values exchanged in pairs: grid (blocks, pairs).
+constexpr int MAX_SWAPS = 9;
+template <typename T>
+struct SwapList {
+    T *a[MAX_SWAPS], *b[MAX_SWAPS];
+    long n;
+};
+
+template <typename T>
+__global__ void k_swap_list(SwapList<T> s) {
+    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= s.n) return;
+    T* a = s.a[blockIdx.y];
+    T* b = s.b[blockIdx.y];
+    const T v = a[idx];
+    a[idx] = b[idx];
+    b[idx] = v;
+}
+
 // ddz_uv (derivatives.f90:214-264): dfdz(k) = (1/dz)(f(k) - f(k-1)), k=1..nz.
 template <typename T>
 __global__ void k_ddz_uv(const T* f, T* out, Geo g, T rdz) {

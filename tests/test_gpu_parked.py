@@ -8,7 +8,7 @@ import lesgo_amd
 
 pytestmark = pytest.mark.gpu
 
-FIELDS = ("u", "v", "w", "p", "RHSx", "RHSz", "dudz", "dvdz", "txz", "tyz", "tzz")
+FIELDS = ("u", "v", "w", "p", "RHSx", "RHSz", "RHSx_f", "dudz", "dvdz", "txz", "tyz", "tzz")
 
 
 def cfg_of(precision="fp64", cfl=False):
@@ -57,3 +57,31 @@ def test_parked_member_keeps_its_fields(precision, cfl):
         c.seed_state(8, 0.1, member=0)
         c.step(2)
         assert_same(want, fields(c, 1))
+
+
+@pytest.mark.parametrize("away", [1, 2])
+@pytest.mark.parametrize("cfl", [False, True])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_parked_member_goes_on_where_it_was(precision, cfl, away):
+    """The buffers that a step exchanges (RHS and RHS_f among them) change
+    places under the parked member too: after an odd and an even number of
+    the others' steps it reads back what it held and steps on as if it had
+    never been away."""
+    with lesgo_amd.Case(cfg_of(precision, cfl)) as a:
+        a.seed_state(4, 0.1)
+        a.step(3)
+        mid = fields(a, 0)
+        a.step(2)
+        end = fields(a, 0)
+    with lesgo_amd.Case(cfg_of(precision, cfl), members=2) as c:
+        for m in range(2):
+            c.seed_state(3 + m, 0.1, member=m)
+        c.set_counters(0, 0)
+        c.step(3)
+        c.set_active(1)
+        c.step(away)
+        assert_same(mid, fields(c, 1))
+        c.step(2)
+        c.set_active(2)
+        c.step_graph(2)
+        assert_same(end, fields(c, 1))
