@@ -1842,7 +1842,7 @@ void Case<T>::materialize(unsigned groups) {
     T* hs[3] = {tmp[6], tmp[7], tmp[8]};
     bool have_gq = false;
     if (groups & SG_DIVT) {
-        // the step keeps no divt spectra (k_spec_ab2 forms divt from the
+        // the step keeps no divt spectra (the column pass forms divt from the
         // stress spectra): the reference's divstress_uv/w on the step's
         // physical stresses (uses spec[0..7] and tmp[0], tmp[2], tmp[4],
         // before the remainders below take tmp)

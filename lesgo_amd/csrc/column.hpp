@@ -23,10 +23,12 @@
 // chain of 2 nz divisions on half the chip's SIMDs.  Measured, those four
 // kernels and this one: 256 x 256 x 192 FP32 454 -> 291 us (4.0 TB/s), FP64
 // 826 -> 540 us (4.3 TB/s); 128^3 FP32 128 -> 45 to 50 us; 64^3 FP32 52 -> 14
-// us; 32^3 FP64 34 -> 9.0 us.  What holds the largest back is address
-// translation: a thread's levels lie a plane apart in every array, so nearly
-// every line of a level misses the CU's first-level TLB (4.9 M misses for 5.3 M
-// lines with 128 bytes a row of the tile, 2.2 M with 256).
+// us; 32^3 FP64 34 -> 9.0 us.  The HBM counters give 1.03 (FP32) and 1.04 (FP64)
+// times those volumes.  What holds the largest back: u* takes a block to 152
+// (FP32) or 153 KB of LDS, so one is on a CU, and its loads, its two sweeps and
+// its stores follow one another with nothing else in flight.  In FP64 one in
+// ten requests also misses the CU's first-level TLB (4.1 M of 39.8 M a launch;
+// FP32 0.07 M of 38.7 M): a thread's levels lie a plane apart in every array.
 #pragma once
 
 #include "pressure.hpp"

@@ -37,13 +37,16 @@ constexpr long HC_CHUNK = 1L << 18;
 constexpr int HC_BUFS = 12;             // chunks in the ring, at most
 constexpr int HC_AHEAD = 3;             // copies in flight
 constexpr int HC_THREADS = 8;
-// Smallest field that takes the ring, in values: 32 MiB of doubles.  Ring and
-// plain copy: 256 x 256 x 192 mixed 7.5 and 19.0 ms, FP64 8.4 and 15.5; 128^3
-// mixed 1.5 and 1.7; 96^3 mixed 0.66 and 0.70; 64^3 FP64 0.31 and 0.43, its
-// first read 1.2 and 0.4.  A destination under 32 MiB is often memory the
-// process has touched before, and what the caller does with it next finds
-// it in the cache of its own core after the plain copy and in eight others'
-// after the ring: four 128^3 fields read and used took 6 ms longer.
+// Smallest field that takes the ring, in values: 32 MiB of doubles.  Reads of
+// four fields in turn, ring and plain copy, ms a field: 256 x 256 x 192 (12.8 M
+// values) mixed 2.1 and 18.9, FP64 3.0 and 10.0; 192^3 (7.2 M) 1.4 and 6.0, 5.3
+// and 6.1; 192 x 144 x 160 (4.5 M) 1.05 and 3.75, 3.3 and 3.8; just below the
+// line, 144 x 144 x 190 (4.0 M), 0.9 and 2.8, 2.2 and 2.6; 128^3 1.5 and 1.9, 0.7
+// and 1.0; 64^3 0.43 and 0.29, 0.6 and 0.4.  The line is not where the reads by
+// themselves cross (near 10^6 values) but above 128^3, where what the program
+// did next cost more than the ring saved: the plain copy leaves a field in
+// the cache of the caller's core, the ring in eight others', and a pass of 128^3
+// steps that reads and converts four fields took 6 ms longer (54 and 60).
 constexpr long HC_MIN = 1L << 22;
 
 class HostCopy {

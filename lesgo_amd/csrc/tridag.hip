@@ -3,8 +3,9 @@
 // a, b, c (lh, ny, nz+1) and an interleaved complex right-hand side r and
 // solution u (ld, ny, nz+1), all FP64 in the reference's column-major layout
 // (C order [nz+1][ny][lh] and [nz+1][ny][ld]).  The time step itself uses
-// the fused k_tridag of pressure.hpp, which assembles the same coefficients
-// from the wavenumbers; this is the drop-in for callers that pass their own.
+// k_column (column.hpp; k_tridag of pressure.hpp on the tallest grids), which
+// assembles the same coefficients from the wavenumbers; this is the drop-in for
+// callers that pass their own.
 #include <mutex>
 #include <string>
 
@@ -34,9 +35,9 @@ constexpr int TRI_STATUS_INTS = 64;
 // stayed at 258 us).  One wave a block puts the systems on all CUs.  The
 // arithmetic and its order are the plain recurrence's.  The whole device call,
 // row at a time and 256 threads a block -> this: 129 x 256 x 193 380 -> 190 us,
-// 65 x 128 x 97 159 -> 91, 33 x 64 x 65 73 -> 50, 9 x 16 x 11 33 -> 33 (of which
-// about 45 are the allocation, the status read and the launch).  Blocks of 4
-// rows 195, of 6 191, of 12 191 us at the first.
+// 65 x 128 x 97 159 -> 93, 33 x 64 x 65 73 -> 48, 9 x 16 x 11 33 -> 31 (in this
+// kernel 131, 36, 25 and 7; the rest is allocations, the status read and the
+// launches).  Blocks of 4 rows 195, of 6 191, of 12 191 us at the first.
 constexpr int TRA_BLK = 8;
 constexpr int TRA_THREADS = 64;
 
