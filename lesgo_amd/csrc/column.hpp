@@ -249,9 +249,9 @@ __global__ void __launch_bounds__(column_max_threads<T>(), sizeof(T) == 4 ? 4 : 
         // fma(fma(-q, bet, t), rb, q) (Markstein).  With rb = 1 / bet correctly
         // rounded q is within 1.5 ulp and the result is t / bet rounded unless
         // t / bet lies within some 2^-52 ulp of the middle between two doubles;
-        // below about 1e-290 the remainder underflows and the result is the
-        // uncorrected q, and an infinite t gives NaN where a division gives
-        // infinity (a run that has diverged).  tests/test_gpu_column_bits.py
+        // below about 1e-290 the remainder can underflow and the correction with
+        // it, and an infinite t gives NaN where a division gives infinity (a
+        // run that has diverged).  tests/test_gpu_column_bits.py
         // compares whole steps with k_tridag's divisions.
         const double c3 = tg.const3;
         const double b_in = -(kxd * kxd + kyd * kyd + 2.0 * c3);
